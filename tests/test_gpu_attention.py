@@ -158,3 +158,24 @@ def test_attention_refusals(backend):
         backend.attention(q, ck, ck, [0], [16], 2, 0.1)
     with pytest.raises(BackendError):  # empty range
         backend.attention(q, ck, ck, [5], [4], 2, 0.1)
+
+
+@pytest.mark.parametrize("n_tok,n_head,n_kv,hd", [(1, 4, 1, 64), (3, 2, 2, 72), (17, 4, 1, 32), (70, 3, 3, 36), (33, 8, 2, 96)],
+                         ids=["4row", "4row_per_row_path", "16row", "16row_per_row_path", "16row_hd96"])
+@pytest.mark.parametrize("length", [1, 15, 33, 127, 128, 129, 256, 257, 385, 512, 600])
+def test_attention_value_tile_edges(backend, oracle, n_tok, n_head, n_kv, hd, length):
+    """The value kernels' tiles of 128 (64 rows and more per K head) and 256 positions: ranges that
+    end around whole tiles, start anywhere in the ring and wrap inside a tile, groups with rows of
+    other ranges and a last group that is not full. Each sum is the reference's chain of fmas, so
+    every output is equal bit for bit."""
+    rng = np.random.default_rng(length * 7 + hd)
+    cap = length + n_tok + 5
+    ck = rng.standard_normal((cap, n_kv * hd)).astype(np.float32)
+    cv = rng.standard_normal((cap, n_kv * hd)).astype(np.float32)
+    q = rng.standard_normal((n_tok, n_head, hd)).astype(np.float32)
+    st = np.full(n_tok, cap // 2 + 3, np.int32)
+    en = (st + length - 1 + np.arange(n_tok)).astype(np.int32)
+    st[n_tok // 2:] += 2 if length > 2 else 0  # rows of one group that start apart
+    scale = float(np.float32(1 / np.sqrt(hd)))
+    o = backend.attention(q, ck, cv, st, en, n_kv, scale)
+    assert bits_equal(o, oracle_attention(oracle, q, ck, cv, st, en, n_kv, scale))

@@ -249,3 +249,21 @@ def test_attention_zero_weight_inf_v_scale(backend, oracle):
     want = oracle_attention(oracle, q, kq, vq, st, en, n_kv, kb, vb, scale)
     assert np.isfinite(want).all()  # the oracle (the reference's skip) stays finite
     assert bits_equal(backend.kvq_attention(q, kq, vq, st, en, n_kv, kb, vb, scale), want)
+
+
+@pytest.mark.parametrize("n_tok,n_head,n_kv,hd,vbits", [(1, 4, 1, 64, 2), (2, 6, 2, 32, 8), (16, 4, 1, 32, 4), (66, 2, 2, 64, 8), (64, 1, 1, 32, 2)])
+@pytest.mark.parametrize("length", [1, 31, 129, 256, 300])
+def test_attention_value_tile_edges(backend, oracle, n_tok, n_head, n_kv, hd, vbits, length):
+    """Ranges around the value kernels' whole tiles (128 and 256 positions) over a ring that wraps,
+    each V width: the reference's chains, equal bit for bit."""
+    rng = np.random.default_rng(length + hd + vbits)
+    cap = length + n_tok + 3
+    k = rng.standard_normal((cap, n_kv, hd)).astype(np.float32)
+    v = rng.standard_normal((cap, n_kv, hd)).astype(np.float32)
+    kq, vq = oracle_cache(oracle, k, v, np.arange(cap, dtype=np.int32), cap, 4, vbits)
+    q = rng.standard_normal((n_tok, n_head, hd)).astype(np.float32)
+    st = np.full(n_tok, cap - 2, np.int32)
+    en = (st + length - 1 + np.arange(n_tok)).astype(np.int32)
+    scale = float(np.float32(1 / np.sqrt(hd)))
+    o = backend.kvq_attention(q, kq, vq, st, en, n_kv, 4, vbits, scale)
+    assert bits_equal(o, oracle_attention(oracle, q, kq, vq, st, en, n_kv, 4, vbits, scale))
