@@ -122,6 +122,13 @@ __device__ __forceinline__ GroupSpan group_span(const AttnArgs &a, int n_tok, in
 typedef float av4 __attribute__((ext_vector_type(4)));  // a native vector: kept in registers when staged
 typedef float av4u __attribute__((ext_vector_type(4), aligned(4)));  // a 16-byte load at a 4-byte boundary
 
+// the workgroup's barrier after LDS writes and reads: global loads stay in flight
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // ---- scores ----
 // K = 1 MFMAs run the 8 lane chains: chain l of every (row, key) pair of a tile is one accumulator
 // register set, and dimension d adds q_d k_d to chain d % 8, each as one fmaf, dimension after
@@ -133,36 +140,44 @@ __device__ __forceinline__ void for_seq(F &&f, std::integer_sequence<int, J...>)
     (f(std::integral_constant<int, J>{}), ...);
 }
 
-// K rows of positions p0 .. p0 + 63 (past hi: hi's row) into dst[64][HD + 4]; NT threads
+// K rows of positions p0 .. p0 + 63 (past hi: hi's row) into dst[64][HD + 4], NT threads: pieces
+// j B .. j B + B - 1 of each thread
 template <int HD, int NT>
-__device__ __forceinline__ void k_tile(const AttnArgs &a, int kh, int p0, int hi, int t, float *dst) {
-    constexpr int Q = HD / 4, N = 64 * Q / NT, B = N > 32 ? N / 2 : N;  // 16-byte pieces per row, per thread, at a time
-    const float *kb = a.k + (int64_t)kh * HD;
-    const int s0 = __builtin_amdgcn_readfirstlane((int)kv_slot(p0, a.cap));
-    const bool whole = p0 + 63 <= hi && s0 + 64 <= a.cap;  // uniform: no wrap, no clamp
-#pragma unroll
-    for (int j = 0; j < N; j += B) {
-        av4 v[B];
-        if (whole) {
+struct KTile {
+    static constexpr int Q = HD / 4, N = 64 * Q / NT, B = N > 32 ? N / 2 : N;  // 16-byte pieces per row, per thread, at a time
+    av4 v[B];
+    __device__ __forceinline__ void load(const AttnArgs &a, int kh, int p0, int hi, int t, int j) {
+        const float *kb = a.k + (int64_t)kh * HD;
+        const int s0 = __builtin_amdgcn_readfirstlane((int)kv_slot(p0, a.cap));
+        if (p0 + 63 <= hi && s0 + 64 <= a.cap) {  // uniform: no wrap, no clamp
 #pragma unroll
             for (int i = 0; i < B; ++i) {
-                const int e = t + (i + j) * NT;
+                const int e = t + (i + j * B) * NT;
                 v[i] = *(const av4 *)(kb + (int64_t)(s0 + e / Q) * a.kv_dim + 4 * (e % Q));
             }
         } else {
 #pragma unroll
             for (int i = 0; i < B; ++i) {
-                const int e = t + (i + j) * NT;
+                const int e = t + (i + j * B) * NT;
                 v[i] = *(const av4 *)(kb + kv_slot(min(p0 + e / Q, hi), a.cap) * a.kv_dim + 4 * (e % Q));
             }
         }
+    }
+    __device__ __forceinline__ void store(int t, int j, float *dst) const {
 #pragma unroll
         for (int i = 0; i < B; ++i) {
-            const int e = t + (i + j) * NT;
+            const int e = t + (i + j * B) * NT;
             *(av4 *)&dst[(e / Q) * (HD + 4) + 4 * (e % Q)] = v[i];
         }
     }
-}
+    __device__ __forceinline__ void copy(const AttnArgs &a, int kh, int p0, int hi, int t, float *dst) {
+#pragma unroll
+        for (int j = 0; j < N / B; ++j) {
+            load(a, kh, p0, hi, t, j);
+            store(t, j, dst);
+        }
+    }
+};
 
 // hsum4_ps's tree over the 8 chains
 __device__ __forceinline__ float chain_tree(float a0, float a1, float a2, float a3, float a4, float a5, float a6, float a7) {
@@ -173,7 +188,8 @@ __device__ __forceinline__ float chain_tree(float a0, float a1, float a2, float 
 // wavefronts. Wavefront w multiplies rows 16 w .. + 15 of the group with a tile of 64 keys by
 // v_mfma_f32_16x16x1: A = q (one register holds 4 dimensions x 16 rows; cbsz = 2 broadcasts the
 // dimension's block to all four), B = K (lane = key), 8 chains x 16 registers of sums, in flight
-// one after another. Two workgroups per CU cover each other's loads.
+// one after another. The next tile's loads are in flight
+// in registers while a tile is multiplied (head sizes up to 128).
 // Bound: one 32-cycle MFMA per dimension and 16 rows x 64 keys.
 template <int HD, int NW>
 __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 192 ? 2 : 1) void attn_scores16_kernel(AttnArgs a, int n_tok) {
@@ -200,9 +216,20 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 192 ? 2 : 1) void attn_sc
         en[i] = g.en;
         out[i] = a.s + (int64_t)g.row * a.max_len - g.st;
     }
-    for (int p0 = sp.lo + (int)blockIdx.z * 64; p0 <= sp.hi; p0 += (int)gridDim.z * 64) {
-        k_tile<HD, 64 * NW>(a, kh, p0, sp.hi, tid, kt);
-        __syncthreads();
+    KTile<HD, 64 * NW> tile;
+    constexpr bool AHEAD = NW == 4 && HD <= 128;  // registers for the next tile beside 8 x 16 sums
+    const int step = (int)gridDim.z * 64;
+    int p0 = sp.lo + (int)blockIdx.z * 64;
+    if (AHEAD && p0 <= sp.hi) tile.load(a, kh, p0, sp.hi, tid, 0);
+    for (; p0 <= sp.hi; p0 += step) {
+        if constexpr (AHEAD) {
+            tile.store(tid, 0, kt);
+            lds_barrier();
+            if (p0 + step <= sp.hi) tile.load(a, kh, p0 + step, sp.hi, tid, 0);
+        } else {
+            tile.copy(a, kh, p0, sp.hi, tid, kt);
+            lds_barrier();
+        }
         av16 acc[8];
 #pragma unroll
         for (int l = 0; l < 8; ++l)
@@ -223,7 +250,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 192 ? 2 : 1) void attn_sc
             const float t = chain_tree(acc[0][r], acc[1][r], acc[2][r], acc[3][r], acc[4][r], acc[5][r], acc[6][r], acc[7][r]);
             if (p >= st[i] && p <= en[i]) out[i][p] = t * a.scale;
         }
-        __syncthreads();
+        lds_barrier();
     }
 }
 
@@ -249,7 +276,8 @@ __global__ __launch_bounds__(128) void attn_scores4_kernel(AttnArgs a, int n_tok
 #pragma unroll
             for (int i = 0; i < NQ; ++i) q[i] = qp[16 * i];
             if (r0 == 0) {
-                k_tile<HD, 64>(a, kh, p0, sp.hi, lane, kt[wave]);
+                KTile<HD, 64> tile;
+                tile.copy(a, kh, p0, sp.hi, lane, kt[wave]);
                 __builtin_amdgcn_wave_barrier();  // the lanes of one wavefront share the tile: its LDS accesses are in order
             }
             av4 acc[8];
@@ -361,28 +389,59 @@ __global__ __launch_bounds__(256) void attn_scores_row_kernel(AttnArgs a, int n_
 // stays in LDS (sized min(max_len, SM_RES) at launch, so short rows leave room for more
 // workgroups per CU) from its one load to its one store: maximum, exponentials, lanes 0..7 of
 // wavefront 0 running the 8 ordered sums, then every value times 1 / sum. Longer rows go
-// through LDS SM_RES positions at a time, the 8 sums carried across the chunks.
+// through LDS SM_RES positions at a time, the 8 sums carried across the chunks. 1024 threads for
+// few rows (decode: a CU holds one row), 256 for prompt batches.
 constexpr int SM_RES = 12288;
 __device__ __forceinline__ float sum8_tree(float v) {  // lanes 0..7: hsum_ps's tree
     v = v + __shfl_xor(v, 4, 8);                       // (v0 + v4), (v1 + v5), ...
     v = v + __shfl_xor(v, 1, 8);
     return v + __shfl_xor(v, 2, 8);  // ((v0 + v4) + (v1 + v5)) + ((v2 + v6) + (v3 + v7))
 }
-__device__ __forceinline__ float lane_sum(const float *e, int ng, int l, float v) {  // v += e[8g + l], g < ng
+// v += e[8g + l], g < ng: 16 values read while the 16 before them are added, one wait per batch
+// (the adds are the bound: 4096 positions are 512 dependent adds)
+__device__ __forceinline__ float lane_sum(const float *e, int ng, int l, float v) {
+    const int n16 = ng & ~15;
+    float t0[16], t1[16];
+    auto read = [&](float *t, int g) {
+        const float *p = e + 8 * g + l;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) t[u] = p[8 * u];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto add = [&](const float *t) {
+        __builtin_amdgcn_s_waitcnt(0xC87F);  // lgkmcnt 8: the next batch's 8 paired reads may be in flight
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v += t[u];
+        __builtin_amdgcn_sched_barrier(0);
+    };
     int g = 0;
-    for (; g + 8 <= ng; g += 8) {
-        float t[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) t[u] = e[8 * (g + u) + l];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v += t[u];
+    if (n16) {
+        read(t0, 0);
+        for (; g + 32 <= n16; g += 32) {
+            read(t1, g + 16);
+            add(t0);
+            read(t0, g + 32 < n16 ? g + 32 : 0);  // past the end: any batch, not added
+            add(t1);
+        }
+        if (g < n16) add(t0);
     }
-    for (; g < ng; ++g) v += e[8 * g + l];
+    for (g = n16; g < ng; ++g) v += e[8 * g + l];
     return v;
 }
-__global__ __launch_bounds__(256) void attn_softmax_kernel(AttnArgs a) {
+template <int NT>
+__device__ __forceinline__ float wg_max(float mx, float *red) {  // every thread of NT calls it
+    for (int o = 1; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) mx = fmaxf(mx, red[w]);
+    return mx;
+}
+template <int NT>
+__global__ __launch_bounds__(NT) void attn_softmax_kernel(AttnArgs a) {
     extern __shared__ float e[];  // min(max_len, SM_RES) values
-    __shared__ float red[4];
+    __shared__ float red[NT / 64];
     __shared__ float total;
     const int row = blockIdx.x, tok = row / a.n_head, tid = threadIdx.x;
     const int n = row_len(a, tok);
@@ -392,21 +451,18 @@ __global__ __launch_bounds__(256) void attn_softmax_kernel(AttnArgs a) {
     const bool resident = n <= SM_RES;
     float mx = -__builtin_inff();
     if (resident) {
-#pragma unroll 8
-        for (int i = tid; i < n; i += 256) {
+#pragma unroll 4
+        for (int i = tid; i < n; i += NT) {
             const float x = s[i];
             e[i] = x;
             mx = fmaxf(mx, x);
         }
     } else {
-        for (int i = tid; i < n; i += 256) mx = fmaxf(mx, s[i]);
+        for (int i = tid; i < n; i += NT) mx = fmaxf(mx, s[i]);
     }
-    for (int o = 1; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    if ((tid & 63) == 0) red[tid >> 6] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    mx = wg_max<NT>(mx, red);
     if (resident) {
-        for (int i = tid; i < n; i += 256) e[i] = i < nv ? exp_neg_ref(e[i] - mx) : expf_ref(e[i] - mx);
+        for (int i = tid; i < n; i += NT) e[i] = i < nv ? exp_neg_ref(e[i] - mx) : expf_ref(e[i] - mx);
         __syncthreads();
         if (tid < 8) {
             float v = sum8_tree(lane_sum(e, nv / 8, tid, 0.0f));
@@ -418,13 +474,13 @@ __global__ __launch_bounds__(256) void attn_softmax_kernel(AttnArgs a) {
         __syncthreads();
         const float sum = total;
         const float inv = 1.0f / sum;
-        for (int i = tid; i < n; i += 256) s[i] = sum > 0.0f ? e[i] * inv : e[i];
+        for (int i = tid; i < n; i += NT) s[i] = sum > 0.0f ? e[i] * inv : e[i];
         return;
     }
     float v = 0.0f;
     for (int c0 = 0; c0 < n; c0 += SM_RES) {
         const int cn = min(SM_RES, n - c0);
-        for (int i = tid; i < cn; i += 256) {
+        for (int i = tid; i < cn; i += NT) {
             const float x = s[c0 + i] - mx;
             const float ev = c0 + i < nv ? exp_neg_ref(x) : expf_ref(x);
             e[i] = ev;
@@ -446,7 +502,7 @@ __global__ __launch_bounds__(256) void attn_softmax_kernel(AttnArgs a) {
     const float sum = total;
     if (sum > 0.0f) {
         const float inv = 1.0f / sum;
-        for (int i = tid; i < n; i += 256) s[i] = s[i] * inv;
+        for (int i = tid; i < n; i += NT) s[i] = s[i] * inv;
     }
 }
 
@@ -588,13 +644,6 @@ struct AvWeights {
     }
 };
 
-// the workgroup's barrier after LDS writes and reads: global loads stay in flight
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // values of prompt batches: grid (K heads, groups of 16 rows, 64-column chunks), 4 chain wavefronts
 // and 8 loading wavefronts. Chain wavefront w sums rows 4 w .. 4 w + 3 of the group over the
 // chunk's 64 columns with v_mfma_f32_4x4x1: its 16 blocks are 16 groups of 4 columns, K = 1 is one
@@ -720,10 +769,12 @@ __global__ __launch_bounds__(768) void attn_values16_kernel(AttnArgs a, int n_to
             for (int g = 0; g < AP_T / 16; g += 2) {
                 read(y, g + 1);
                 __builtin_amdgcn_s_waitcnt(0xC57F);  // lgkmcnt 5: y's reads may be in flight
+                __builtin_amdgcn_sched_barrier(0);
                 sum(x);
                 if (g + 2 < AP_T / 16) {
                     read(x, g + 2);
                     __builtin_amdgcn_s_waitcnt(0xC57F);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
                 sum(y);
             }
@@ -864,10 +915,12 @@ __global__ __launch_bounds__(320) void attn_values4_kernel(AttnArgs a, int n_tok
             for (int i = 0; i < AD_T / 32; i += 2) {
                 read(y, i + 1);
                 __builtin_amdgcn_s_waitcnt(0xCA7F);  // lgkmcnt 10: y's reads may be in flight
+                __builtin_amdgcn_sched_barrier(0);
                 sum(x);
                 if (i + 2 < AD_T / 32) {
                     read(x, i + 2);
                     __builtin_amdgcn_s_waitcnt(0xCA7F);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
                 sum(y);
             }
@@ -952,7 +1005,10 @@ hipError_t launch_attention(const AttnArgs &a, int n_tok, hipStream_t s) {
         default: scores_launch<256>(a, n_tok, s); break;
         }
     }
-    attn_softmax_kernel<<<n_tok * a.n_head, 256, (size_t)std::min(a.max_len, SM_RES) * 4, s>>>(a);
+    const int rows = n_tok * a.n_head;
+    const size_t lds = (size_t)std::min(a.max_len, SM_RES) * 4;
+    if (rows <= 256) attn_softmax_kernel<1024><<<rows, 1024, lds, s>>>(a);
+    else attn_softmax_kernel<256><<<rows, 256, lds, s>>>(a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     return launch_attention_values(a, n_tok, s);  // 4 chains per lane from 64 rows per K / V head

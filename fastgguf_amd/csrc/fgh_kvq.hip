@@ -42,102 +42,164 @@ struct SignTable {
 };
 __constant__ SignTable kvq_sign = SignTable();
 
-// Lloyd-Max centroids of N(0, 1) (kvq_c4 / kvq_c2, 3356-3359) and the midpoints between
-// neighbours, in float as kvq_enc4 / kvq_enc2 form them
-__constant__ float kvq_c4[16] = {-2.7326f, -2.0690f, -1.6181f, -1.2562f, -0.9424f, -0.6568f, -0.3881f, -0.1284f,
-                                 0.1284f,  0.3881f,  0.6568f,  0.9424f,  1.2562f,  1.6181f,  2.0690f,  2.7326f};
-__constant__ float kvq_c2[4] = {-1.5104f, -0.4528f, 0.4528f, 1.5104f};
-
 __device__ __forceinline__ int64_t slot_of(int p, int cap) { return (int64_t)(((p % cap) + cap) % cap); }
 
-// the rotation (or its inverse) of x[0..hd) in LDS; 256 threads, all of them call it
-__device__ void rotate_lds(float *x, int hd, bool inverse) {
-    const int tid = threadIdx.x;
+// The rotation (or its inverse) of one row in one wavefront: lane l holds values l + 64 e (hd 32:
+// lanes 0..31, value l). Butterflies up to 32 apart are lane exchanges, wider ones stay in the
+// lane; every value sees the reference's additions (lower: a + b, upper: a - b).
+constexpr int KVQ_E = 4;  // hd <= 256
+__device__ __forceinline__ void rotate_wave(float (&x)[KVQ_E], int hd, bool inverse) {
+    const int lane = threadIdx.x & 63, ne = hd < 64 ? 1 : hd / 64;
     if (!inverse)
-        for (int i = tid; i < hd; i += 256) x[i] = x[i] * kvq_sign.v[i];
-    __syncthreads();
-    for (int len = 1; len < hd; len <<= 1) {
-        for (int t = tid; t < hd / 2; t += 256) {
-            const int i = (t / len) * 2 * len + (t % len);
-            const float a = x[i], b = x[i + len];
-            x[i] = a + b;
-            x[i + len] = a - b;
+#pragma unroll
+        for (int e = 0; e < KVQ_E; ++e) x[e] = x[e] * kvq_sign.v[lane + 64 * e];
+#pragma unroll
+    for (int len = 1; len < 64; len <<= 1) {
+        if (len < hd) {
+#pragma unroll
+            for (int e = 0; e < KVQ_E; ++e)
+                if (e < ne) {
+                    const float o = __shfl_xor(x[e], len, 64);
+                    x[e] = lane & len ? o - x[e] : x[e] + o;
+                }
         }
-        __syncthreads();
+    }
+    if (hd >= 128) {
+#pragma unroll
+        for (int e = 0; e < KVQ_E; e += 2) {
+            const float p = x[e], q = x[e + 1];
+            x[e] = p + q;
+            x[e + 1] = p - q;
+        }
+    }
+    if (hd >= 256) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float p = x[e], q = x[e + 2];
+            x[e] = p + q;
+            x[e + 2] = p - q;
+        }
     }
     const float inv = 1.0f / sqrtf((float)hd);
-    for (int i = tid; i < hd; i += 256) x[i] = inverse ? x[i] * inv * kvq_sign.v[i] : x[i] * inv;
-    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < KVQ_E; ++e) x[e] = inverse ? x[e] * inv * kvq_sign.v[lane + 64 * e] : x[e] * inv;
+}
+__device__ __forceinline__ void row_load(float (&x)[KVQ_E], const float *src, int hd) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int e = 0; e < KVQ_E; ++e) x[e] = lane + 64 * e < hd ? src[lane + 64 * e] : 0.0f;
 }
 
+// the number of midpoints below u: the first code whose upper midpoint u does not pass
+// (kvq_enc4 / kvq_enc2; a NaN passes none)
 __device__ __forceinline__ uint32_t code4(float u) {
     uint32_t c = 0;
-    while (c < 15 && u > (kvq_c4[c] + kvq_c4[c + 1]) * 0.5f) ++c;
+#pragma unroll
+    for (int i = 0; i < 15; ++i) c += u > (kvq_centroid4(i) + kvq_centroid4(i + 1)) * 0.5f ? 1u : 0u;
     return c;
 }
 __device__ __forceinline__ uint32_t code2(float u) {
     uint32_t c = 0;
-    while (c < 3 && u > (kvq_c2[c] + kvq_c2[c + 1]) * 0.5f) ++c;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) c += u > (kvq_centroid2(i) + kvq_centroid2(i + 1)) * 0.5f ? 1u : 0u;
     return c;
 }
 
-// store: grid (tokens, K / V heads, 2: K then V), 256 threads. Rotates the head slice of the
-// token's new K or V row and writes its record into slot pos % cap (kvq_quant_slice 3415-3444).
+// sum += p[0], p[1], .. p[n - 1] in order (n a multiple of 32, p in LDS, 16-byte aligned): 32 values
+// read while the 32 before them are added, one wait per batch. All lanes run the same sum.
+__device__ __forceinline__ float ordered_sum(const float *p, int n, float sum) {
+    typedef float kv4 __attribute__((ext_vector_type(4)));
+    kv4 t0[8], t1[8];
+    auto read = [&](kv4 *t, int i) {
+        const kv4 *q = (const kv4 *)(p + i);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) t[u] = q[u];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto add = [&](const kv4 *t) {
+        __builtin_amdgcn_s_waitcnt(0xC87F);  // lgkmcnt 8: the next batch may be in flight
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            sum += t[u].x;
+            sum += t[u].y;
+            sum += t[u].z;
+            sum += t[u].w;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (n <= 0) return sum;
+    read(t0, 0);
+    int i = 0;
+    for (; i + 64 <= n; i += 64) {
+        read(t1, i + 32);
+        add(t0);
+        read(t0, i + 64 < n ? i + 64 : 0);  // past the end: any batch, not added
+        add(t1);
+    }
+    if (i < n) add(t0);
+    return sum;
+}
+
+// store: grid (tokens, K / V heads, 2: K then V), one wavefront. Rotates the head slice of the
+// token's new K or V row and writes its record into slot pos % cap (kvq_quant_slice 3415-3444):
+// each lane encodes its own values, and the lanes of a 32-bit word combine theirs by exchanges.
 // The reference writes token after token: where two tokens of a call share a slot, only the
 // later one writes.
-__global__ __launch_bounds__(256) void kvq_store_kernel(KvqStoreArgs a, int n_tok) {
-    __shared__ float x[256];
-    __shared__ float sc[2];
-    const int tok = blockIdx.x, kh = blockIdx.y, isv = blockIdx.z, tid = threadIdx.x, hd = a.hd;
+__global__ __launch_bounds__(64) void kvq_store_kernel(KvqStoreArgs a, int n_tok) {
+    __shared__ __attribute__((aligned(16))) float sq[256];
+    const int tok = blockIdx.x, kh = blockIdx.y, isv = blockIdx.z, lane = threadIdx.x, hd = a.hd;
+    float x[KVQ_E];
+    row_load(x, (isv ? a.v : a.k) + (size_t)tok * a.stride + (size_t)kh * hd, hd);
     const int64_t my_slot = slot_of(a.pos[tok], a.cap);
     bool later = false;
-    for (int t = tok + 1 + tid; t < n_tok; t += 256) later |= slot_of(a.pos[t], a.cap) == my_slot;
-    if (__syncthreads_or(later)) return;  // the whole workgroup
+    for (int t = tok + 1 + lane; t < n_tok; t += 64) later |= slot_of(a.pos[t], a.cap) == my_slot;
+    if (__builtin_amdgcn_ballot_w64(later)) return;  // the whole wavefront
     const int bits = isv ? a.vbits : a.kbits;
-    const float *src = (isv ? a.v : a.k) + (size_t)tok * a.stride + (size_t)kh * hd;
-    for (int i = tid; i < hd; i += 256) x[i] = src[i];
-    __syncthreads();
-    rotate_lds(x, hd, false);
-    if (tid == 0) {
-        float s;
-        if (bits == 8) {
-            float amax = 0.0f;
-            for (int i = 0; i < hd; ++i) amax = fmaxf(amax, fabsf(x[i]));
-            s = amax / 127.0f;
-        } else {
-            float ss = 0.0f;
-            for (int i = 0; i < hd; ++i) ss = ss + x[i] * x[i];
-            s = sqrtf(ss / (float)hd);
-        }
-        sc[0] = s;
-        sc[1] = s > 0.0f ? 1.0f / s : 0.0f;
+    rotate_wave(x, hd, false);
+    float s;
+    if (bits == 8) {
+        float amax = 0.0f;
+#pragma unroll
+        for (int e = 0; e < KVQ_E; ++e)
+            if (lane + 64 * e < hd) amax = fmaxf(amax, fabsf(x[e]));
+        for (int o = 1; o < 64; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+        s = amax / 127.0f;
+    } else {  // the squares in parallel, their sum in order
+#pragma unroll
+        for (int e = 0; e < KVQ_E; ++e)
+            if (lane + 64 * e < hd) sq[lane + 64 * e] = x[e] * x[e];
+        __syncthreads();
+        s = sqrtf(ordered_sum(sq, hd, 0.0f) / (float)hd);
     }
-    __syncthreads();
-    const float inv = sc[1];
+    const float inv = s > 0.0f ? 1.0f / s : 0.0f;
     const int rec = 4 + hd * bits / 8;
     uint8_t *dst = (isv ? a.vq : a.kq) + my_slot * (int64_t)(a.n_head_kv * rec) + (int64_t)kh * rec;
-    if (tid == 0) *(float *)dst = sc[0];
+    if (lane == 0) *(float *)dst = s;
     uint32_t *words = (uint32_t *)(dst + 4);
-    const int per = 32 / bits;  // codes per 32-bit word
-    for (int w = tid; w < hd / per; w += 256) {
-        uint32_t v = 0;
-        for (int j = 0; j < per; ++j) {
-            const float u = x[w * per + j] * inv;
-            const uint32_t c = bits == 8 ? (uint32_t)(uint8_t)(int8_t)(int)rintf(u) : bits == 4 ? code4(u) : code2(u);
-            v |= c << (bits * j);
-        }
-        words[w] = v;
+    const int per = 32 / bits;  // codes per 32-bit word: per adjacent lanes
+#pragma unroll
+    for (int e = 0; e < KVQ_E; ++e) {
+        if (64 * e >= hd) break;  // uniform
+        const float u = x[e] * inv;
+        uint32_t v = bits == 8 ? (uint32_t)(uint8_t)(int8_t)(int)rintf(u) : bits == 4 ? code4(u) : code2(u);
+        v <<= bits * (lane & (per - 1));
+        for (int o = 1; o < per; o <<= 1) v |= (uint32_t)__shfl_xor((int)v, o, 64);
+        if ((lane & (per - 1)) == 0 && lane + 64 * e < hd) words[(lane + 64 * e) / per] = v;
     }
 }
 
-// rows of hd values rotated (inverse = false) or rotated back: one workgroup per row
-__global__ __launch_bounds__(256) void kvq_rotate_kernel(const float *in, float *out, int hd, bool inverse) {
-    __shared__ float x[256];
-    const size_t base = (size_t)blockIdx.x * hd;
-    for (int i = threadIdx.x; i < hd; i += 256) x[i] = in[base + i];
-    __syncthreads();
-    rotate_lds(x, hd, inverse);
-    for (int i = threadIdx.x; i < hd; i += 256) out[base + i] = x[i];
+// rows of hd values rotated (inverse = false) or rotated back: one wavefront per row, 4 rows per
+// workgroup
+__global__ __launch_bounds__(256) void kvq_rotate_kernel(const float *in, float *out, int hd, int rows, bool inverse) {
+    const int row = (int)blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= rows) return;
+    float x[KVQ_E];
+    row_load(x, in + (size_t)row * hd, hd);
+    rotate_wave(x, hd, inverse);
+#pragma unroll
+    for (int e = 0; e < KVQ_E; ++e)
+        if (lane + 64 * e < hd) out[(size_t)row * hd + lane + 64 * e] = x[e];
 }
 
 __device__ __forceinline__ int kvq_row_len(const KvqAttnArgs &a, int tok) {
@@ -187,7 +249,7 @@ __global__ __launch_bounds__(256) void kvq_scores_kernel(KvqAttnArgs a, int n_to
         const KvqRow g = kvq_group_row(a, n_tok, R, grp, kh, r);
         q[r][x] = g.en >= g.st ? a.qr[(size_t)g.row * hd + x] : 0.0f;
     }
-    if (tid < 16) c4[tid] = kvq_c4[tid];
+    if (tid < 16) c4[tid] = kvq_centroid4(tid);
     __syncthreads();
     const int rec = 4 + hd * a.kbits / 8;
     for (int p = lo + (int)blockIdx.x * 256 + tid; p <= hi; p += (int)gridDim.x * 256) {
@@ -227,51 +289,67 @@ __global__ __launch_bounds__(256) void kvq_scores_kernel(KvqAttnArgs a, int n_to
     }
 }
 
-// softmax_inplace over each row's scores, then each weight times its position's V scale
+// softmax_inplace over each row's scores, then each weight times its position's V scale. The sum is
+// one ordered chain per row: about 5 cycles per position out of LDS. 1024 threads for few rows
+// (decode: a CU holds one row), 256 for prompt batches.
 constexpr int KVQ_RES = 12288;
-__global__ __launch_bounds__(256) void kvq_softmax_kernel(KvqAttnArgs a) {
-    extern __shared__ float e[];  // min(max_len, KVQ_RES) values: rows up to that length stay in LDS
-    __shared__ float red[4];
+template <int NT>
+__global__ __launch_bounds__(NT) void kvq_softmax_kernel(KvqAttnArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float e[];  // min(max_len, KVQ_RES) values: rows up to that length stay in LDS
+    __shared__ float red[NT / 64];
     __shared__ float total;
     const int row = blockIdx.x, tok = row / a.n_head, h = row - tok * a.n_head, tid = threadIdx.x;
     const int n = kvq_row_len(a, tok);
     if (n == 0) return;
     float *s = a.s + (size_t)row * a.max_len;
+    const bool resident = n <= KVQ_RES;
     float mx = -__builtin_inff();
-    for (int i = tid; i < n; i += 256) mx = fmaxf(mx, s[i]);
+#pragma unroll 4
+    for (int i = tid; i < n; i += NT) {
+        const float x = s[i];
+        if (resident) e[i] = x;
+        mx = fmaxf(mx, x);
+    }
     for (int o = 1; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
     if ((tid & 63) == 0) red[tid >> 6] = mx;
     __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    const bool resident = n <= KVQ_RES;
-    for (int i = tid; i < n; i += 256) {
-        const float ev = expf_ref(s[i] - mx);
-        if (resident) e[i] = ev;
-        else s[i] = ev;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) mx = fmaxf(mx, red[w]);
+    for (int i = tid; i < n; i += NT) {
+        if (resident) e[i] = expf_ref(e[i] - mx);
+        else s[i] = expf_ref(s[i] - mx);
     }
     __syncthreads();
-    if (tid == 0) {  // the sum in order: 32 values loaded ahead of their adds
+    if (tid < 64) {
         float sum = 0.0f;
-        const float *src = resident ? e : s;
         int i = 0;
-        for (; i + 32 <= n; i += 32) {
-            float t[32];
+        if (resident) {
+            sum = ordered_sum(e, n & ~31, sum);
+            for (i = n & ~31; i < n; ++i) sum += e[i];
+        } else {  // 32 values loaded ahead of their adds
+            for (; i + 32 <= n; i += 32) {
+                float t[32];
 #pragma unroll
-            for (int u = 0; u < 32; ++u) t[u] = src[i + u];
+                for (int u = 0; u < 32; ++u) t[u] = s[i + u];
 #pragma unroll
-            for (int u = 0; u < 32; ++u) sum += t[u];
+                for (int u = 0; u < 32; ++u) sum += t[u];
+            }
+            for (; i < n; ++i) sum += s[i];
         }
-        for (; i < n; ++i) sum += src[i];
-        total = sum;
+        if (tid == 0) total = sum;
     }
     __syncthreads();
     const float sum = total, inv = 1.0f / sum;
     const int kvh = h / (a.n_head / a.n_head_kv), rec = 4 + a.hd * a.vbits / 8;
-    for (int i = tid; i < n; i += 256) {
+    const uint8_t *vr = a.vq + (int64_t)kvh * rec;
+    const int64_t stride = (int64_t)a.n_head_kv * rec;
+    const int64_t s0 = slot_of(a.st[tok], a.cap);
+#pragma unroll 4
+    for (int i = tid; i < n; i += NT) {  // n <= cap: the ring wraps at most once
         const float ev = resident ? e[i] : s[i];
         const float w = sum > 0.0f ? ev * inv : ev;
-        const float sv =
-            *(const float *)(a.vq + slot_of(a.st[tok] + i, a.cap) * (int64_t)(a.n_head_kv * rec) + (int64_t)kvh * rec);
+        const int64_t sl = s0 + i < a.cap ? s0 + i : s0 + i - a.cap;
+        const float sv = *(const float *)(vr + sl * stride);
         // kvq_axpy_v skips a zero weight (fastgguf.c:4829-4831): stored as 0, never 0 * s_V, so a V
         // record whose scale is inf or NaN adds nothing where the reference adds nothing
         s[i] = w == 0.0f ? 0.0f : w * sv;
@@ -284,7 +362,7 @@ hipError_t launch_kvq_store(const KvqStoreArgs &a, int n_tok, hipStream_t s) {
     if (n_tok < 1 || a.hd < 32 || a.hd > 256 || (a.hd & (a.hd - 1)) || (a.kbits != 4 && a.kbits != 8) ||
         (a.vbits != 2 && a.vbits != 4 && a.vbits != 8) || a.n_head_kv < 1 || a.n_head_kv > 65535)
         return hipErrorInvalidValue;
-    kvq_store_kernel<<<dim3((unsigned)n_tok, (unsigned)a.n_head_kv, 2), 256, 0, s>>>(a, n_tok);
+    kvq_store_kernel<<<dim3((unsigned)n_tok, (unsigned)a.n_head_kv, 2), 64, 0, s>>>(a, n_tok);
     return hipGetLastError();
 }
 
@@ -294,21 +372,23 @@ hipError_t launch_kvq_attention(const KvqAttnArgs &a, int n_tok, hipStream_t s) 
         (a.vbits != 2 && a.vbits != 4 && a.vbits != 8) || a.n_head_kv < 1 || a.n_head % a.n_head_kv != 0 ||
         a.max_len < 1 || rows > 65535)
         return hipErrorInvalidValue;
-    kvq_rotate_kernel<<<rows, 256, 0, s>>>(a.q, a.qr, a.hd, false);
+    kvq_rotate_kernel<<<(rows + 3) / 4, 256, 0, s>>>(a.q, a.qr, a.hd, rows, false);
     const int rows_kv = n_tok * (a.n_head / a.n_head_kv);
     const unsigned kb = (unsigned)std::min((a.max_len + 255) / 256, 1024);
     if (rows_kv >= 16)
         kvq_scores_kernel<16><<<dim3(kb, (unsigned)((rows_kv + 15) / 16), (unsigned)a.n_head_kv), 256, 0, s>>>(a, n_tok);
     else
         kvq_scores_kernel<4><<<dim3(kb, (unsigned)((rows_kv + 3) / 4), (unsigned)a.n_head_kv), 256, 0, s>>>(a, n_tok);
-    kvq_softmax_kernel<<<rows, 256, (size_t)std::min(a.max_len, KVQ_RES) * 4, s>>>(a);
+    const size_t lds = (size_t)std::min(a.max_len, KVQ_RES) * 4;
+    if (rows <= 256) kvq_softmax_kernel<1024><<<rows, 1024, lds, s>>>(a);
+    else kvq_softmax_kernel<256><<<rows, 256, lds, s>>>(a);
     AttnArgs v{nullptr, a.orot, nullptr, nullptr, a.s, a.st, a.en, a.n_head, a.n_head_kv, a.hd,
                a.n_head_kv * a.hd, a.cap, a.max_len, 1.0f};
     v.vq = a.vq;  // the value chains decode the V records' codes themselves
     v.vbits = a.vbits;
     hipError_t e = launch_attention_values(v, n_tok, s);
     if (e != hipSuccess) return e;
-    kvq_rotate_kernel<<<rows, 256, 0, s>>>(a.orot, a.o, a.hd, true);
+    kvq_rotate_kernel<<<(rows + 3) / 4, 256, 0, s>>>(a.orot, a.o, a.hd, rows, true);
     return hipGetLastError();
 }
 
