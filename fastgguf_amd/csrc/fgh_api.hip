@@ -398,6 +398,27 @@ static int prompt_gemm(fgh_ctx *c, const fgh_tensor *t, const float *X, int64_t 
     return prompt_gemm_into(c, t, X, ldx, Y, ldy, T, (uint8_t *)c->gq.p, ds, dm);
 }
 
+// The matmuls of several tokens that the reference runs token by token, in its row kernels' orders:
+// the kernels that share a matrix's weights between tokens, and the scratch bytes they need. Their
+// outputs are the per-token decode kernels' bit for bit, so a call whose scratch is not at hand
+// (a graph capture before any eager call) takes those.
+static bool tokens_path(const fgh_ctx *c, const fgh_tensor *t, int64_t ldx, int T) {
+    if (T < 2) return false;
+    if (q16_rows(t->type)) return fgh::rowg_pays((int)t->type, t->order, t->groups, t->nb, T, c->num_cu);
+    if (!fgh::fl_kind((int)t->type)) return false;
+    // the float kernels address X and a step of a matrix by 32-bit offsets
+    return 4 * ((T - 1) * ldx + t->cols) <= 0x7fffffff && t->gpm * fgh::FL_TILE <= 0x7fffffff &&
+           fgh::fl_matmul_pays((int)t->type, t->rows * t->n_mats, (int)t->cols, T, c->num_cu);
+}
+static size_t tokens_bytes(const fgh_tensor *t, int T) { return q16_rows(t->type) ? fgh::rowg_act_bytes(t->nb, T) : 0; }
+static int tokens_into(fgh_ctx *c, const fgh_tensor *t, const float *X, int64_t ldx, float *Y, int64_t ldy, int T,
+                       uint8_t *act) {
+    const fgh::RowgArgs r{t->dev, X, Y, act, t->rows, t->gpm, t->groups, ldx, ldy, t->nb, T};
+    HIP_TRY(c, fgh::fl_kind((int)t->type) ? fgh::launch_fl_matmul((int)t->type, r, c->num_cu, c->stream)
+                                          : fgh::launch_rowg((int)t->type, t->order, r, c->num_cu, c->stream));
+    return FGH_OK;
+}
+
 // host-synchronous and allocating calls cannot be recorded into a graph
 #define NO_CAPTURE(c) \
     do { \
@@ -713,9 +734,16 @@ int fgh_matmul_dev(fgh_ctx *c, const fgh_tensor *t, const float *X, int ldx, flo
     INJECT(c);
     HIP_TRY(c, hipSetDevice(c->device));
     // nb >= 8: the prompt GEMMs (matmul 3018-3031) on int8 MFMA for Q4_K, Q6_K, Q8_0 and the nibble
-    // types Q4_0 / Q4_1 / Q5_0 / Q5_1; Q5_K, IQ4_NL, Q2_K, Q3_K and IQ4_XS, which have no GEMM in the
-    // reference, run the per-token decode kernels as its matmul does
+    // types Q4_0 / Q4_1 / Q5_0 / Q5_1; smaller batches, and the types without a GEMM in the reference,
+    // keep the order of its token by token calls
     if (prompt_gemm_bytes(c, t, nb)) return prompt_gemm(c, t, X, ldx, Y, ldy, nb, nullptr, nullptr);
+    if (tokens_path(c, t, ldx, nb)) {
+        const size_t need = tokens_bytes(t, nb);
+        if (!c->capturing || need <= c->gq.cap) {
+            if ((rc = grow(c, c->gq, need))) return rc;
+            return tokens_into(c, t, X, ldx, Y, ldy, nb, (uint8_t *)c->gq.p);
+        }
+    }
     float *ys[1] = {Y};
     return matvec_launch(c, 1, &t, X, ldx, ys, ldy, nb, nullptr, nullptr);
 }
@@ -738,6 +766,9 @@ int fgh_matmul_dev_noalloc(fgh_ctx *c, const fgh_tensor *t, const float *X, int 
     INJECT(c);
     HIP_TRY(c, hipSetDevice(c->device));
     if (gemm) return prompt_gemm_into(c, t, X, ldx, Y, ldy, nb, (uint8_t *)c->noalloc, nullptr, nullptr);
+    // the several-token kernels that need scratch stay out: without a prompt GEMM a call here uses no
+    // shared memory, so such calls may overlap
+    if (tokens_path(c, t, ldx, nb) && !tokens_bytes(t, nb)) return tokens_into(c, t, X, ldx, Y, ldy, nb, nullptr);
     float *ys[1] = {Y};
     return matvec_launch(c, 1, &t, X, ldx, ys, ldy, nb, nullptr, nullptr);
 }

@@ -122,13 +122,6 @@ __device__ __forceinline__ GroupSpan group_span(const AttnArgs &a, int n_tok, in
 typedef float av4 __attribute__((ext_vector_type(4)));  // a native vector: kept in registers when staged
 typedef float av4u __attribute__((ext_vector_type(4), aligned(4)));  // a 16-byte load at a 4-byte boundary
 
-// the workgroup's barrier after LDS writes and reads: global loads stay in flight
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // ---- scores ----
 // K = 1 MFMAs run the 8 lane chains: chain l of every (row, key) pair of a tile is one accumulator
 // register set, and dimension d adds q_d k_d to chain d % 8, each as one fmaf, dimension after

@@ -29,6 +29,9 @@
 // Tiles (upload, fl_relayout_kernel): step s of row tile t of matrix m at
 // ((m * steps + s) * tiles per matrix + t) * 1 KB, lane L's 16 bytes at 16 L; values past the
 // row's end and rows past the matrix's end are zeros (never on a chain).
+#include <algorithm>
+#include <type_traits>
+
 #include "fgh_internal.h"
 
 namespace fgh {
@@ -305,6 +308,305 @@ hipError_t launch_fl_relayout(int type, const uint8_t *src, uint8_t *dst, int64_
     const int64_t units = total / 16, want = (units + 255) / 256;
     const unsigned grid = (unsigned)(want < 65536 ? want : 65536);
     fl_relayout_kernel<<<grid, 256, 0, s>>>(type, src, dst, rows, cols, steps, gpm, units);
+    return hipGetLastError();
+}
+
+// ---- several tokens (matmul): the same chains on fp32 MFMAs of K = 1 ----
+// The reference multiplies float matrices token by token (matmul, fastgguf.c:3004-3017), each chain
+// an ordered run of fmas. v_mfma_f32_*x1 adds one product to every sum of its tile, each as one
+// fmaf (subnormals, infinities and NaN included: measured on 8 M products), so a chain of rank-1
+// updates over the values in order is the reference's chain for 16 rows x 16 tokens at once.
+// F32 / F16: v_mfma_f32_16x16x1 with its 4 blocks as 4 chains: lane 16 b + i of A holds row i's
+// value of chain 4 h + b, lane 16 b + t of B token t's activation; a lane then holds all chains of
+// 4 rows x 1 token, so the final tree needs no exchange. BF16 has one chain per row: A = tokens
+// (one register holds 4 positions x 16 tokens, the position's block broadcast), B = 64 rows.
+// Workgroup = 4 wavefronts on 4 row tiles, sharing stages of 256 NT / (values) activations in LDS,
+// loaded a stage ahead; grid.y = chunks of NT groups of 16 tokens.
+// Bound: MFMA (one per value, 16 x 16 outputs and 4 chains: 128 fmas per cycle and CU) from about
+// 16 tokens, below that the weight stream (F32, F16) or the dependent MFMAs (BF16).
+typedef float fm4 __attribute__((ext_vector_type(4)));
+typedef float fm4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float fm16 __attribute__((ext_vector_type(16)));
+
+struct FlMmArgs {
+    const uint8_t *W;
+    const float *X;
+    float *Y;
+    int64_t rows, gpm, ldx, ldy;  // rows and tiles per matrix
+    int n, nst, T;                // values per row, steps, tokens
+    uint32_t wpm;                 // wavefront tiles per matrix
+    int64_t groups;               // wavefront tiles
+    uint32_t xbytes;              // X up to its last value (below 2 GiB)
+};
+
+// NT groups of 16 tokens per wavefront, SB steps of 64 values per stage (NT SB = 4: 16 KB)
+template <int TYPE, int NT>
+__global__ __launch_bounds__(256, NT == 4 ? 1 : 2) void fl_mm_kernel(FlMmArgs a) {
+    using F = Fl<TYPE>;
+    constexpr int SB = 4 / NT, HN = F::C / 4, VQ = F::V / 4, R = TYPE == T_F32 ? 4 : 8, TW = 16 / F::TR;
+    static_assert(F::CV == 64 && R % SB == 0, "stage geometry");
+    __shared__ __attribute__((aligned(16))) float xs[2][4096];  // [step][group][h][u / 4][lane][u % 4]
+    const int tid = threadIdx.x, l = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = a.n, nst = a.nst, tok0 = (int)blockIdx.y * 16 * NT;
+    const int64_t wt = (int64_t)blockIdx.x * 4 + wave;
+    const bool live = wt < a.groups;
+    const uint32_t tc = (uint32_t)(live ? wt : a.groups - 1), mi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tc / a.wpm)), wl = tc - mi * a.wpm;
+    const int b = l >> 4, i = l & 15;
+    // A: row i of the wavefront's 16 rows: row i % TR of tile TW wl + i / TR
+    const uint32_t tile = wl * TW + (uint32_t)(i / F::TR);
+    const bool rlive = live && tile < (uint32_t)a.gpm;
+    const size_t sstride = (size_t)a.gpm * FL_TILE;
+    const uint8_t *M0 = a.W + (size_t)mi * nst * sstride;  // the matrix
+    // a lane whose tile does not exist reads past the buffer's end: zeros, no access
+    const uint32_t off = rlive ? tile * FL_TILE + 16 * (F::C * (i % F::TR) + b) : 0x80000000u;
+    auto wload = [&](int s, uint4 (&w)[HN]) {
+        const BufRes r = buf_res(M0 + (size_t)min(s, nst - 1) * sstride, live && s < nst ? (uint32_t)sstride : 0u);
+#pragma unroll
+        for (int h = 0; h < HN; ++h) w[h] = bld16(r, off + 64 * h);
+    };
+    uint4 ring[R][HN];
+#pragma unroll
+    for (int q = 0; q < R; ++q) wload(q, ring[q]);
+    // activations: thread (t, q) takes values 4 q .. + 3 of token t of each group and step
+    const int xt = tid >> 4, xq = tid & 15;
+    fm4 xr[4];
+    // one buffer over all tokens; a quad that is not whole lies past the chains (the scalar tail reads
+    // X itself) and, like one past the row, is out of the buffer's range: zeros, no access, no branch
+    const BufRes xb = buf_res((const uint8_t *)a.X, a.xbytes);
+    auto xload = [&](int st) {  // stage st: steps SB st .. + SB - 1
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int s = SB * st + j / NT, tok = min(tok0 + 16 * (j % NT) + xt, a.T - 1), e = 64 * s + 4 * xq;
+            const uint4 v = bld16(xb, e + 4 <= n ? 4u * ((uint32_t)tok * (uint32_t)a.ldx + (uint32_t)e) : 0x80000000u);
+            xr[j] = (fm4){__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)};
+        }
+    };
+    auto xstore = [&](int st) {
+        float *d = xs[st & 1];
+        const int k0 = (4 * xq) % F::C, u = (4 * xq) / F::C;  // 4 adjacent chains of value u
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                d[(((j * HN) + (k0 >> 2)) * VQ + (u >> 2)) * 256 + (16 * c + xt) * 4 + (u & 3)] = xr[j][c];
+    };
+    fm16 acc[NT][HN];
+#pragma unroll
+    for (int g = 0; g < NT; ++g)
+#pragma unroll
+        for (int h = 0; h < HN; ++h)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[g][h][e] = 0.0f;
+    const int nstage = (nst + SB - 1) / SB;
+    xload(0);
+    xstore(0);
+    if (nstage > 1) xload(1);
+    lds_barrier();
+    // a step: its activations read, its weights converted (each into a register of its own: an MFMA in
+    // flight holds its operands), then the MFMAs; all: every value of the step is on its chain
+    auto step = [&](auto all, int s0, int q, uint4 (&w)[HN]) {  // step s0 + q, s0 a multiple of R
+        constexpr bool whole = decltype(all)::value;
+        const int s = s0 + q;
+        const float *x = xs[(s / SB) & 1] + (size_t)(q % SB) * NT * HN * VQ * 256 + 4 * l;
+        if (q % SB == 0) {  // a new stage
+            if (s / SB + 1 < nstage) xstore(s / SB + 1);
+            xload(min(s / SB + 2, nstage - 1));
+        }
+        fm4 xv[NT][HN][VQ];
+#pragma unroll
+        for (int g = 0; g < NT; ++g)
+#pragma unroll
+            for (int h = 0; h < HN; ++h)
+#pragma unroll
+                for (int q = 0; q < VQ; ++q) xv[g][h][q] = *(const fm4 *)(x + ((g * HN + h) * VQ + q) * 256);
+        float wv[HN][F::V];
+#pragma unroll
+        for (int h = 0; h < HN; ++h)
+#pragma unroll
+            for (int u = 0; u < F::V; ++u) wv[h][u] = fl_val<TYPE>(w[h], u);
+        wload(s + R, w);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < F::V; ++u)
+#pragma unroll
+            for (int h = 0; h < HN; ++h)
+                if (whole || on_chain<TYPE>(s, u, 4 * h, n)) {  // the 4 chains of h agree
+#pragma unroll
+                    for (int g = 0; g < NT; ++g)
+                        acc[g][h] = __builtin_amdgcn_mfma_f32_16x16x1f32(wv[h][u], xv[g][h][u >> 2][u & 3], acc[g][h], 0, 0, 0);
+                }
+        if (q % SB == SB - 1) lds_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int s0 = 0;
+    for (; 64 * (s0 + R) <= n; s0 += R) {  // whole rounds: straight-line code
+#pragma unroll
+        for (int q = 0; q < R; ++q) step(std::true_type{}, s0, q, ring[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+        if (s0 + q < nst) step(std::false_type{}, s0, q, ring[q]);  // uniform over the workgroup
+    // lane (q, t): rows 4 q + r, token t; register 4 b + r of acc[.][h] is chain 4 h + b
+#pragma unroll
+    for (int g = 0; g < NT; ++g) {
+        const int tok = tok0 + 16 * g + i;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                v[k] = acc[g][k >> 2][4 * (k & 3) + r];
+                if constexpr (TYPE == T_F32) v[k] = v[k] + acc[g][2 + (k >> 2)][4 * (k & 3) + r];  // s0_k + s1_k
+            }
+            float y = ((v[0] + v[4]) + (v[1] + v[5])) + ((v[2] + v[6]) + (v[3] + v[7]));
+            const int64_t row = (int64_t)wl * 16 + 4 * b + r;
+            if (live && row < a.rows && tok < a.T) {
+                const int t0 = TYPE == T_F32 ? 16 * (n / 16) + (n % 16 >= 8 ? 8 : 0) : 8 * (n / 8);
+                const uint8_t *T0 = M0 + (size_t)(row / F::TR) * FL_TILE;
+                for (int e = t0; e < n; ++e)
+                    y = __builtin_fmaf(fl_val_at<TYPE>(T0, sstride, (int)(row % F::TR), e), a.X[(size_t)tok * a.ldx + e], y);
+                a.Y[(size_t)tok * a.ldy + (int64_t)mi * a.rows + row] = y;
+            }
+        }
+    }
+}
+
+// BF16: a wavefront holds 64 rows (lane = row: the decode tile) x 16 tokens, stages of 128 values of
+// the tokens in LDS ([value / 4][lane]: lane 16 c + t of an A register is position 4 q + c of token t)
+__global__ __launch_bounds__(256) void fl_mm_bf16_kernel(FlMmArgs a) {
+    using F = Fl<T_BF16>;
+    constexpr int SV = 128, SS = SV / F::CV, R = 16, TB = 16;  // values and steps per stage, ring, tokens
+    static_assert(R == SS, "a ring round is a stage");
+    __shared__ __attribute__((aligned(16))) float xs[2][SV * TB];
+    const int tid = threadIdx.x, l = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = a.n, nst = a.nst, tok0 = (int)blockIdx.y * TB;
+    const int64_t wt = (int64_t)blockIdx.x * 4 + wave;
+    const bool live = wt < a.groups;
+    const uint32_t tc = (uint32_t)(live ? wt : a.groups - 1), mi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tc / a.wpm)), wl = tc - mi * a.wpm;
+    const size_t sstride = (size_t)a.gpm * FL_TILE;
+    const uint8_t *T0 = a.W + (size_t)mi * nst * sstride + (size_t)wl * FL_TILE;
+    const int nstage = (n + SV - 1) / SV;
+    uint4 ring[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) ring[q] = fl_load(T0 + (size_t)min(q, nst - 1) * sstride, (uint32_t)l, live && q < nst);
+    const BufRes xb = buf_res((const uint8_t *)a.X, a.xbytes);  // past the row: out of range, zeros
+    fm4 xr[2];  // thread (t, q): values 4 q .. + 3 of tokens t and t + 8
+    auto xload = [&](int st) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int t = (tid >> 5) + 8 * j, e = SV * st + 4 * (tid & 31);
+            const uint32_t o = 4u * ((uint32_t)min(tok0 + t, a.T - 1) * (uint32_t)a.ldx + (uint32_t)e);
+            if (n % 4 == 0 || st + 1 < nstage) {  // uniform: whole quads
+                const uint4 v = bld16(xb, e < n ? o : 0x80000000u);
+                xr[j] = (fm4){__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)};
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    xr[j][c] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xb, e + c < n ? (int)(o + 4 * c) : (int)0x80000000u, 0, 0));
+            }
+        }
+    };
+    auto xstore = [&](int st) {
+        float *d = xs[st & 1] + 64 * (tid & 31) + (tid >> 5);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) d[16 * c + 8 * j] = xr[j][c];
+    };
+    fm16 acc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+    xload(0);
+    xstore(0);
+    if (nstage > 1) xload(1);
+    lds_barrier();
+    auto run = [&](auto all, int st) {  // a stage; all: every value of it exists (no test per value)
+        constexpr bool whole = decltype(all)::value;
+        if (st + 1 < nstage) xstore(st + 1);
+        xload(min(st + 2, nstage - 1));
+        const float *x = xs[st & 1] + l;
+        const int cnt = min(SV, n - st * SV);
+#pragma unroll
+        for (int q = 0; q < SS; ++q) {
+            // the step's operands in registers of their own, then its MFMAs
+            float w[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) w[u] = fl_val<T_BF16>(ring[q], u);
+            const float x0 = x[64 * (2 * q)], x1 = x[64 * (2 * q + 1)];
+            const int s = SS * st + q;
+            ring[q] = fl_load(T0 + (size_t)min(s + R, nst - 1) * sstride, (uint32_t)l, live && s + R < nst);
+            __builtin_amdgcn_sched_barrier(0);
+#define FL_B(u, X, J) \
+    if (whole || 8 * q + u < cnt) acc = __builtin_amdgcn_mfma_f32_16x16x1f32(X, w[u], acc, 2, J, 0);
+            FL_B(0, x0, 0) FL_B(1, x0, 1) FL_B(2, x0, 2) FL_B(3, x0, 3)
+            FL_B(4, x1, 0) FL_B(5, x1, 1) FL_B(6, x1, 2) FL_B(7, x1, 3)
+#undef FL_B
+        }
+        lds_barrier();
+    };
+    int st = 0;
+    for (; SV * (st + 1) <= n; ++st) run(std::true_type{}, st);
+    if (st < nstage) run(std::false_type{}, st);
+    // register 4 b + r: token 4 (l / 16) + r of row 16 b + l % 16
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const int tok = tok0 + 4 * (l >> 4) + (e & 3);
+        const int64_t row = (int64_t)wl * 64 + 16 * (e >> 2) + (l & 15);
+        if (live && row < a.rows && tok < a.T) a.Y[(size_t)tok * a.ldy + (int64_t)mi * a.rows + row] = acc[e];
+    }
+}
+
+// groups of 16 tokens per wavefront: the most that still fill the compute units; F32's 16 chains
+// leave room for one
+static int fl_mm_nt(int type, int64_t groups, int tg, int num_cu) {
+    int nt = type != T_F16 ? 1 : tg >= 3 ? 4 : tg;
+    while (nt > 1 && (groups + 3) / 4 * ((tg + nt - 1) / nt) < num_cu * 3 / 4) nt >>= 1;
+    return nt;
+}
+// Whether these kernels take less time than the per-token decode launches, from what both measured on
+// MI355X (us, n values a row): the decode launches 3 + (F32 0.5, F16 0.13 below 8 M weights and 0.19
+// above) per token and million weights, BF16 the larger of 0.0113 n and 0.155 per token and
+// million; these 4 + (F32 0.48, F16 0.375 per group of tokens) per 64 values, BF16 0.026 per
+// value, times the rounds of wavefronts (a wavefront walks its whole rows). 14336 x 2048, 64
+// tokens: F32 998 -> 72, F16 444 -> 52, BF16 312 -> 58; 4096 x 4096: 533 -> 38, 195 -> 31, 152 -> 107.
+bool fl_matmul_pays(int type, int64_t rows, int n, int T, int num_cu) {
+    const double mw = (double)rows * n * 1e-6;
+    const int tg = (T + 15) / 16;
+    const int64_t groups = (rows + (type == T_BF16 ? 63 : 15)) / (type == T_BF16 ? 64 : 16);
+    const int nt = fl_mm_nt(type, groups, tg, num_cu);
+    const double rounds = (double)((groups * ((tg + nt - 1) / nt) + 4 * num_cu - 1) / (4 * num_cu));
+    if (type == T_BF16) return std::max(0.0113 * n, 0.155 * T * mw) > 1.15 * (2 + 0.026 * n * rounds);
+    const double before = 3 + T * mw * (type == T_F32 ? 0.5 : mw < 8 ? 0.13 : 0.19);
+    return before > 1.15 * (4 + (type == T_F32 ? 0.48 : 0.375 * nt) * ((n + 63) / 64) * rounds);
+}
+template <int TYPE>
+static hipError_t fl_mm_launch(const FlMmArgs &a, int num_cu, hipStream_t s) {
+    const int tg = (a.T + 15) / 16, nt = fl_mm_nt(TYPE, a.groups, tg, num_cu);
+    const dim3 g((unsigned)((a.groups + 3) / 4), (unsigned)((tg + nt - 1) / nt));
+    if constexpr (TYPE != T_F32) {
+        if (nt == 4) fl_mm_kernel<TYPE, 4><<<g, 256, 0, s>>>(a);
+        if (nt == 2) fl_mm_kernel<TYPE, 2><<<g, 256, 0, s>>>(a);
+    }
+    if (nt == 1) fl_mm_kernel<TYPE, 1><<<g, 256, 0, s>>>(a);
+    return hipGetLastError();
+}
+hipError_t launch_fl_matmul(int type, const RowgArgs &r, int num_cu, hipStream_t s) {
+    if (!fl_kind(type) || r.nb < 1 || r.T < 1 || r.T > 64 || r.groups < 1 || r.gpm < 1 || r.groups % r.gpm != 0 ||
+        r.gpm * fl_tile_rows(type) < r.rows || !r.W || !r.X || !r.Y)
+        return hipErrorInvalidValue;
+    const int64_t mats = r.groups / r.gpm;
+    const int tw = type == T_BF16 ? 1 : 16 / fl_tile_rows(type);
+    FlMmArgs a{r.W, r.X, r.Y, r.rows, r.gpm, r.ldx, r.ldy, r.nb, (r.nb + fl_step_elems(type) - 1) / fl_step_elems(type), r.T,
+               (uint32_t)((r.gpm + tw - 1) / tw), 0, 0};
+    a.groups = mats * a.wpm;
+    const int64_t xb = 4 * ((r.T - 1) * r.ldx + r.nb);
+    if (xb > 0x7fffffff) return hipErrorInvalidValue;
+    a.xbytes = (uint32_t)xb;
+    if ((a.groups + 3) / 4 > 0x7fffffff || r.gpm * FL_TILE > 0x7fffffff) return hipErrorInvalidValue;
+    if (type == T_F32) return fl_mm_launch<T_F32>(a, num_cu, s);
+    if (type == T_F16) return fl_mm_launch<T_F16>(a, num_cu, s);
+    const unsigned wg = (unsigned)((a.groups + 3) / 4);
+    fl_mm_bf16_kernel<<<dim3(wg, (unsigned)((a.T + 15) / 16)), 256, 0, s>>>(a);
     return hipGetLastError();
 }
 

@@ -112,6 +112,13 @@ __device__ __forceinline__ uint32_t pack_q(int a, int b, int c, int d) {
     return (uint32_t)(a & 0xFF) | ((uint32_t)(b & 0xFF) << 8) | ((uint32_t)(c & 0xFF) << 16) | ((uint32_t)(d & 0xFF) << 24);
 }
 
+// the workgroup's barrier after LDS writes and reads: global loads stay in flight
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // ---- cross-lane helpers (DPP: no LDS traffic) ----
 __device__ __forceinline__ int dpp_xor1(int v) {  // quad_perm [1,0,3,2]
     return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);
@@ -624,6 +631,22 @@ struct KvqAttnArgs {
     float scale;
 };
 hipError_t launch_kvq_attention(const KvqAttnArgs &a, int n_tok, hipStream_t s);
+
+// matmul of 2..64 tokens in the decode kernels' orders: Q4_K and Q5_K (fgh_rowg.hip), F32, F16 and
+// BF16 (fgh_float.hip, no scratch)
+struct RowgArgs {
+    const uint8_t *W;  // tile layout
+    const float *X;    // tokens, stride ldx
+    float *Y;          // Y[tok * ldy + row]
+    uint8_t *act;      // scratch (rowg_act_bytes), or null
+    int64_t rows, gpm, groups, ldx, ldy;
+    int nb, T;         // blocks (float types: values) per row, tokens
+};
+size_t rowg_act_bytes(int nb, int T);
+bool rowg_pays(int type, int order, int64_t groups, int nb, int T, int num_cu);  // faster than the per-token launches
+bool fl_matmul_pays(int type, int64_t rows, int n, int T, int num_cu);
+hipError_t launch_rowg(int type, int order, const RowgArgs &r, int num_cu, hipStream_t s);
+hipError_t launch_fl_matmul(int type, const RowgArgs &r, int num_cu, hipStream_t s);
 
 // prompt-batch Q4_K GEMM (fgh_gemm.hip): 1..64 tokens, weights in the Q4_K decode layout
 struct GemmArgs {

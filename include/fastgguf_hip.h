@@ -162,8 +162,9 @@ FGH_API int fgh_matvec_multi(fgh_ctx *ctx, int n, const fgh_tensor *const *t, co
 
 /* ---- matmul: replaces matmul (fastgguf.c:3004) for nb <= 64 tokens ----
  * Y[tok * ldy + r] = dot(W[r], Q8(X[tok * ldx ...])). nb >= 8 runs the int8 MFMA prompt GEMM
- * (the role of gemm_kquant 2818 / gemm_q32 2981); nb < 8 runs the decode kernel per token, as the
- * reference does for repacked tensors (3006-3009). */
+ * (the role of gemm_kquant 2818 / gemm_q32 2981); nb < 8 gives the decode kernel's outputs per token, as
+ * the reference does for repacked tensors (3006-3009): so do types without a prompt GEMM at every nb.
+ * Where it is faster, Q4_K, Q5_K and the float types share a matrix's weights between the tokens. */
 FGH_API int fgh_matmul(fgh_ctx *ctx, const fgh_tensor *t, const float *X, int ldx, float *Y, int ldy, int nb);
 
 /* ---- MoE FFN: replaces moe_ffn (fastgguf.c:4588) for n_tok tokens ----
