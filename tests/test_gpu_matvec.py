@@ -357,3 +357,18 @@ def test_copy_d2d(backend):
     assert np.array_equal(a, b)
     backend.dev_free(src)
     backend.dev_free(dst)
+
+
+@pytest.mark.parametrize("rows", [(1,), (5, 3, 65528), (65536,), (65537,), (40000, 30000)], ids=str)
+def test_host_staging_edges(backend, oracle, rows):
+    """Host matvecs whose outputs together just fit the pinned staging memory (65,536 floats) and just do
+    not, one and several tensors; the same call twice, with other activations."""
+    cols = 32
+    ws = [S.weights(S.T_Q8_0, r, cols, 60 + r) for r in rows]
+    ts = [backend.upload(S.T_Q8_0, cols, w) for w in ws]
+    for seed in (1, 2):
+        x = S.activations(cols, seed)
+        for w, y in zip(ws, backend.matvec_multi(ts, x)):
+            assert bits_equal(y, oracle.matvec(S.T_Q8_0, w, cols, x))
+    for t in ts:
+        t.free()
