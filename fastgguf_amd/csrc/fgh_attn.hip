@@ -223,19 +223,17 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 192 ? 2 : 1) void attn_sc
             tile.copy(a, kh, p0, sp.hi, tid, kt);
             lds_barrier();
         }
-        av16 acc[8];
+        av16 acc[8], zero;  // a chain's first MFMA adds to a constant 0
 #pragma unroll
-        for (int l = 0; l < 8; ++l)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[l][i] = 0.0f;
+        for (int i = 0; i < 16; ++i) zero[i] = 0.0f;
         const float *kr = kt + lane * (HD + 4);
         for_seq([&](auto d) {
             constexpr int D = decltype(d)::value;
             const av4 k = *(const av4 *)(kr + 4 * D);
-            acc[4 * (D & 1) + 0] = __builtin_amdgcn_mfma_f32_16x16x1f32(q[D], k.x, acc[4 * (D & 1) + 0], 2, 0, 0);
-            acc[4 * (D & 1) + 1] = __builtin_amdgcn_mfma_f32_16x16x1f32(q[D], k.y, acc[4 * (D & 1) + 1], 2, 1, 0);
-            acc[4 * (D & 1) + 2] = __builtin_amdgcn_mfma_f32_16x16x1f32(q[D], k.z, acc[4 * (D & 1) + 2], 2, 2, 0);
-            acc[4 * (D & 1) + 3] = __builtin_amdgcn_mfma_f32_16x16x1f32(q[D], k.w, acc[4 * (D & 1) + 3], 2, 3, 0);
+            acc[4 * (D & 1) + 0] = __builtin_amdgcn_mfma_f32_16x16x1f32(q[D], k.x, D < 2 ? zero : acc[4 * (D & 1) + 0], 2, 0, 0);
+            acc[4 * (D & 1) + 1] = __builtin_amdgcn_mfma_f32_16x16x1f32(q[D], k.y, D < 2 ? zero : acc[4 * (D & 1) + 1], 2, 1, 0);
+            acc[4 * (D & 1) + 2] = __builtin_amdgcn_mfma_f32_16x16x1f32(q[D], k.z, D < 2 ? zero : acc[4 * (D & 1) + 2], 2, 2, 0);
+            acc[4 * (D & 1) + 3] = __builtin_amdgcn_mfma_f32_16x16x1f32(q[D], k.w, D < 2 ? zero : acc[4 * (D & 1) + 3], 2, 3, 0);
         }, std::make_integer_sequence<int, HD / 4>{});
 #pragma unroll
         for (int r = 0; r < 16; ++r) {

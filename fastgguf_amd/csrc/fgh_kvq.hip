@@ -319,6 +319,20 @@ __global__ __launch_bounds__(NT) void kvq_softmax_kernel(KvqAttnArgs a) {
         if (resident) e[i] = expf_ref(e[i] - mx);
         else s[i] = expf_ref(s[i] - mx);
     }
+    // the V scales of this thread's first positions, in flight while the sum runs; n <= cap: the ring
+    // wraps at most once
+    const int kvh = h / (a.n_head / a.n_head_kv), rec = 4 + a.hd * a.vbits / 8;
+    const uint8_t *vr = a.vq + (int64_t)kvh * rec;
+    const int64_t stride = (int64_t)a.n_head_kv * rec;
+    const int64_t s0 = slot_of(a.st[tok], a.cap);
+    auto vscale = [&](int i) {
+        const int64_t sl = s0 + i < a.cap ? s0 + i : s0 + i - a.cap;
+        return *(const float *)(vr + sl * stride);
+    };
+    constexpr int PF = 4;
+    float pf[PF];
+#pragma unroll
+    for (int k = 0; k < PF; ++k) pf[k] = vscale(min(tid + k * NT, n - 1));
     __syncthreads();
     if (tid < 64) {
         float sum = 0.0f;
@@ -340,20 +354,17 @@ __global__ __launch_bounds__(NT) void kvq_softmax_kernel(KvqAttnArgs a) {
     }
     __syncthreads();
     const float sum = total, inv = 1.0f / sum;
-    const int kvh = h / (a.n_head / a.n_head_kv), rec = 4 + a.hd * a.vbits / 8;
-    const uint8_t *vr = a.vq + (int64_t)kvh * rec;
-    const int64_t stride = (int64_t)a.n_head_kv * rec;
-    const int64_t s0 = slot_of(a.st[tok], a.cap);
-#pragma unroll 4
-    for (int i = tid; i < n; i += NT) {  // n <= cap: the ring wraps at most once
+    auto weigh = [&](int i, float sv) {
         const float ev = resident ? e[i] : s[i];
         const float w = sum > 0.0f ? ev * inv : ev;
-        const int64_t sl = s0 + i < a.cap ? s0 + i : s0 + i - a.cap;
-        const float sv = *(const float *)(vr + sl * stride);
         // kvq_axpy_v skips a zero weight (fastgguf.c:4829-4831): stored as 0, never 0 * s_V, so a V
         // record whose scale is inf or NaN adds nothing where the reference adds nothing
         s[i] = w == 0.0f ? 0.0f : w * sv;
-    }
+    };
+#pragma unroll
+    for (int k = 0; k < PF; ++k)
+        if (tid + k * NT < n) weigh(tid + k * NT, pf[k]);
+    for (int i = tid + PF * NT; i < n; i += NT) weigh(i, vscale(i));
 }
 
 }  // namespace
