@@ -229,63 +229,107 @@ __device__ __forceinline__ KvqRow kvq_group_row(const KvqAttnArgs &a, int n_tok,
 
 // scores: grid (key blocks, groups of R rows, K / V heads), 256 threads; thread = one key of the
 // group's union for its R rows: each record's codes are loaded and looked up once for R chains
-// in kvq_dot_k's order, then times s, times scale. R = 16 for prompt batches.
+// in kvq_dot_k's order, then times s, times scale. R = 16 for prompt batches. R = 4 (decode): each
+// wavefront rotates one of the rows itself, while its keys' records are on their way: 10.8 us at 32
+// heads, 4096 positions, hd 128, against 9.7 and a rotation launch of 4.0. (With 16 rows per group
+// every key block would rotate 4 per wavefront.) A record's words are requested 8 ahead of their
+// use. Bound: latency, one or two wavefronts per CU and SIMD; twice the workgroups of 128 threads
+// took 11.5 us against 11.3.
 template <int R>
 __global__ __launch_bounds__(256) void kvq_scores_kernel(KvqAttnArgs a, int n_tok) {
     __shared__ float q[R][256];
     __shared__ float c4[16];
     const int grp = blockIdx.y, kh = blockIdx.z, tid = threadIdx.x, hd = a.hd;
-    int lo = 0x7fffffff, hi = -0x7fffffff;
-    for (int r = 0; r < R; ++r) {
-        const KvqRow g = kvq_group_row(a, n_tok, R, grp, kh, r);
-        if (g.en >= g.st) {
-            lo = min(lo, g.st);
-            hi = max(hi, g.en);
-        }
+    // every wavefront finds the group's ranges for itself: lane r (mod R) reads row r's, one round of
+    // loads, and lane exchanges reduce them. R = 4: its own row of q is on its way meanwhile
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    float x[KVQ_E] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (R == 4) {
+        const int G = a.n_head / a.n_head_kv, j = grp * R + wave, t = j / G;
+        if (t < n_tok) row_load(x, a.q + ((size_t)t * a.n_head + kh * G + (j - t * G)) * hd, hd);
     }
+    const KvqRow mine = kvq_group_row(a, n_tok, R, grp, kh, lane & (R - 1));
+    const bool ok = mine.en >= mine.st;
+    int lo = ok ? mine.st : 0x7fffffff, hi = ok ? mine.en : -0x7fffffff;
+    for (int o = 1; o < R; o <<= 1) {
+        lo = min(lo, __shfl_xor(lo, o, 64));
+        hi = max(hi, __shfl_xor(hi, o, 64));
+    }
+    lo = __builtin_amdgcn_readfirstlane(lo);
+    hi = __builtin_amdgcn_readfirstlane(hi);
     if (hi < lo) return;
-    for (int i = tid; i < R * hd; i += 256) {
-        const int r = i / hd, x = i - r * hd;
-        const KvqRow g = kvq_group_row(a, n_tok, R, grp, kh, r);
-        q[r][x] = g.en >= g.st ? a.qr[(size_t)g.row * hd + x] : 0.0f;
+    KvqRow rows[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        rows[r] = KvqRow{__builtin_amdgcn_readlane(mine.row, r), __builtin_amdgcn_readlane(mine.st, r), __builtin_amdgcn_readlane(mine.en, r)};
+    constexpr int CW = 8;
+    const int rec = 4 + hd * a.kbits / 8, nw = hd * a.kbits / 32;
+    const uint32_t *w = nullptr;
+    uint32_t cur[CW], nxt[CW];
+    float s = 0.0f;
+    auto words = [&](uint32_t (&d)[CW], int c) {  // words c .. c + 7, the last one past the record's end
+#pragma unroll
+        for (int u = 0; u < CW; ++u) d[u] = w[min(c + u, nw - 1)];
+    };
+    auto start = [&](int p) {  // key p's scale and first words (past hi: hi's)
+        const uint8_t *rp = a.kq + slot_of(min(p, hi), a.cap) * (int64_t)(a.n_head_kv * rec) + (int64_t)kh * rec;
+        w = (const uint32_t *)(rp + 4);
+        s = *(const float *)rp;
+        words(cur, 0);
+    };
+    int p = lo + (int)blockIdx.x * 256 + tid;
+    start(p);
+    if constexpr (R == 4) {
+        rotate_wave(x, hd, false);
+#pragma unroll
+        for (int e = 0; e < KVQ_E; ++e) q[wave][lane + 64 * e] = x[e];  // past hd, and rows without a range: not used
+    } else {
+        for (int i = tid; i < R * hd; i += 256) {
+            const int r = i / hd, x = i - r * hd;
+            const KvqRow g = kvq_group_row(a, n_tok, R, grp, kh, r);
+            q[r][x] = g.en >= g.st ? a.qr[(size_t)g.row * hd + x] : 0.0f;
+        }
     }
     if (tid < 16) c4[tid] = kvq_centroid4(tid);
     __syncthreads();
-    const int rec = 4 + hd * a.kbits / 8;
-    for (int p = lo + (int)blockIdx.x * 256 + tid; p <= hi; p += (int)gridDim.x * 256) {
-        const uint8_t *rp = a.kq + slot_of(p, a.cap) * (int64_t)(a.n_head_kv * rec) + (int64_t)kh * rec;
-        const float s = *(const float *)rp;
-        const uint32_t *w = (const uint32_t *)(rp + 4);
+    for (; p <= hi; p += (int)gridDim.x * 256) {
         float acc[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) acc[r] = 0.0f;
-        if (a.kbits == 8) {
-            for (int i = 0; i < hd; i += 4) {
-                const uint32_t v = w[i / 4];
+        for (int c = 0; c < nw; c += CW) {
+            if (c + CW < nw) words(nxt, c + CW);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float c = (float)(int8_t)(v >> (8 * j));
+            for (int u = 0; u < CW; ++u) {
+                if (c + u >= nw) break;  // uniform
+                const uint32_t v = cur[u];
+                if (a.kbits == 8) {
+                    const int i = 4 * (c + u);
 #pragma unroll
-                    for (int r = 0; r < R; ++r) acc[r] = __builtin_fmaf(q[r][i + j], c, acc[r]);
+                    for (int j = 0; j < 4; ++j) {
+                        const float k = (float)(int8_t)(v >> (8 * j));
+#pragma unroll
+                        for (int r = 0; r < R; ++r) acc[r] = __builtin_fmaf(q[r][i + j], k, acc[r]);
+                    }
+                } else {
+                    const int i = 8 * (c + u);
+#pragma unroll
+                    for (int j = 0; j < 8; j += 2) {
+                        const float clo = c4[(v >> (4 * j)) & 15], chi = c4[(v >> (4 * j + 4)) & 15];
+#pragma unroll
+                        for (int r = 0; r < R; ++r)
+                            acc[r] = acc[r] + __builtin_fmaf(q[r][i + j], clo, q[r][i + j + 1] * chi);
+                    }
                 }
             }
-        } else {
-            for (int i = 0; i < hd; i += 8) {
-                const uint32_t v = w[i / 8];
 #pragma unroll
-                for (int j = 0; j < 8; j += 2) {
-                    const float clo = c4[(v >> (4 * j)) & 15], chi = c4[(v >> (4 * j + 4)) & 15];
-#pragma unroll
-                    for (int r = 0; r < R; ++r)
-                        acc[r] = acc[r] + __builtin_fmaf(q[r][i + j], clo, q[r][i + j + 1] * chi);
-                }
-            }
+            for (int u = 0; u < CW; ++u) cur[u] = nxt[u];
         }
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const KvqRow g = kvq_group_row(a, n_tok, R, grp, kh, r);
+            const KvqRow g = rows[r];
             if (p >= g.st && p <= g.en) a.s[(size_t)g.row * a.max_len + (p - g.st)] = acc[r] * s * a.scale;
         }
+        if (p + (int)gridDim.x * 256 <= hi) start(p + (int)gridDim.x * 256);
     }
 }
 
@@ -315,7 +359,10 @@ __global__ __launch_bounds__(NT) void kvq_softmax_kernel(KvqAttnArgs a) {
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < NT / 64; ++w) mx = fmaxf(mx, red[w]);
-    for (int i = tid; i < n; i += NT) {
+    // decode rows: the first NT exponentials here, the others while wavefront 0 sums those (20.2 ->
+    // 17.4 us, 32 rows of 4096 positions)
+    const bool split = NT == 1024 && resident && n > NT;
+    for (int i = tid; i < (split ? NT : n); i += NT) {
         if (resident) e[i] = expf_ref(e[i] - mx);
         else s[i] = expf_ref(s[i] - mx);
     }
@@ -334,12 +381,20 @@ __global__ __launch_bounds__(NT) void kvq_softmax_kernel(KvqAttnArgs a) {
 #pragma unroll
     for (int k = 0; k < PF; ++k) pf[k] = vscale(min(tid + k * NT, n - 1));
     __syncthreads();
+    float head = 0.0f;  // wavefront 0: the sum of the first NT
+    if (split) {
+        if (tid < 64) head = ordered_sum(e, NT, 0.0f);
+        else
+            for (int i = NT + tid - 64; i < n; i += NT - 64) e[i] = expf_ref(e[i] - mx);
+        __syncthreads();
+    }
     if (tid < 64) {
-        float sum = 0.0f;
+        float sum = head;
         int i = 0;
         if (resident) {
-            sum = ordered_sum(e, n & ~31, sum);
-            for (i = n & ~31; i < n; ++i) sum += e[i];
+            const int from = split ? NT : 0, to = n & ~31;
+            sum = ordered_sum(e + from, to - from, sum);
+            for (i = to; i < n; ++i) sum += e[i];
         } else {  // 32 values loaded ahead of their adds
             for (; i + 32 <= n; i += 32) {
                 float t[32];
@@ -383,12 +438,12 @@ hipError_t launch_kvq_attention(const KvqAttnArgs &a, int n_tok, hipStream_t s) 
         (a.vbits != 2 && a.vbits != 4 && a.vbits != 8) || a.n_head_kv < 1 || a.n_head % a.n_head_kv != 0 ||
         a.max_len < 1 || rows > 65535)
         return hipErrorInvalidValue;
-    kvq_rotate_kernel<<<(rows + 3) / 4, 256, 0, s>>>(a.q, a.qr, a.hd, rows, false);
     const int rows_kv = n_tok * (a.n_head / a.n_head_kv);
     const unsigned kb = (unsigned)std::min((a.max_len + 255) / 256, 1024);
-    if (rows_kv >= 16)
+    if (rows_kv >= 16) {
+        kvq_rotate_kernel<<<(rows + 3) / 4, 256, 0, s>>>(a.q, a.qr, a.hd, rows, false);
         kvq_scores_kernel<16><<<dim3(kb, (unsigned)((rows_kv + 15) / 16), (unsigned)a.n_head_kv), 256, 0, s>>>(a, n_tok);
-    else
+    } else
         kvq_scores_kernel<4><<<dim3(kb, (unsigned)((rows_kv + 3) / 4), (unsigned)a.n_head_kv), 256, 0, s>>>(a, n_tok);
     const size_t lds = (size_t)std::min(a.max_len, KVQ_RES) * 4;
     if (rows <= 256) kvq_softmax_kernel<1024><<<rows, 1024, lds, s>>>(a);

@@ -267,3 +267,25 @@ def test_attention_value_tile_edges(backend, oracle, n_tok, n_head, n_kv, hd, vb
     scale = float(np.float32(1 / np.sqrt(hd)))
     o = backend.kvq_attention(q, kq, vq, st, en, n_kv, 4, vbits, scale)
     assert bits_equal(o, oracle_attention(oracle, q, kq, vq, st, en, n_kv, 4, vbits, scale))
+
+
+@pytest.mark.parametrize("hd,kbits", [(32, 4), (64, 8), (128, 4), (256, 8)])
+@pytest.mark.parametrize("length", [1024, 1025, 1055, 1056, 1987, 2049])
+def test_attention_decode_long_row_edges(backend, oracle, hd, kbits, length):
+    """Decode rows around the softmax's first 1024 positions and its batches of 32, the scores'
+    records from half a round of words (hd 32) to eight, three rows per K / V head over a wrapping
+    ring: equal bit for bit."""
+    rng = np.random.default_rng(length + hd)
+    n_kv, n_head, cap = 2, 6, length + 2
+    kq = rng.integers(0, 256, (cap, n_kv * rec_bytes(hd, kbits)), dtype=np.uint8)
+    vq = rng.integers(0, 256, (cap, n_kv * rec_bytes(hd, 4)), dtype=np.uint8)
+    for cache, bits, top in ((kq, kbits, 0.02), (vq, 4, 2.0)):  # positive finite scales
+        for h in range(n_kv):
+            at = h * rec_bytes(hd, bits)
+            cache[:, at:at + 4] = rng.uniform(top / 4, top, (cap, 1)).astype(np.float32).view(np.uint8)
+    q = rng.standard_normal((1, n_head, hd)).astype(np.float32)
+    st = np.full(1, cap - 5, np.int32)
+    en = (st + length - 1).astype(np.int32)
+    scale = float(np.float32(1 / np.sqrt(hd)))
+    o = backend.kvq_attention(q, kq, vq, st, en, n_kv, kbits, 4, scale)
+    assert bits_equal(o, oracle_attention(oracle, q, kq, vq, st, en, n_kv, kbits, 4, scale))
