@@ -289,3 +289,21 @@ def test_attention_decode_long_row_edges(backend, oracle, hd, kbits, length):
     scale = float(np.float32(1 / np.sqrt(hd)))
     o = backend.kvq_attention(q, kq, vq, st, en, n_kv, kbits, 4, scale)
     assert bits_equal(o, oracle_attention(oracle, q, kq, vq, st, en, n_kv, kbits, 4, scale))
+
+
+@pytest.mark.parametrize("cap", [63, 511, 512, 513, 700])
+@pytest.mark.parametrize("vbits", [2, 4, 8])
+def test_attention_prompt_gathered_scales(backend, oracle, cap, vbits):
+    """A prompt batch whose V scales just fit the scratch they are gathered into (cap 512: 2 heads x
+    cap values in 32 rows x 32) and just do not, over a wrapping ring: equal bit for bit."""
+    rng = np.random.default_rng(cap + vbits)
+    n_tok, n_kv, hd = 16, 2, 32
+    k = rng.standard_normal((cap, n_kv, hd)).astype(np.float32)
+    v = (rng.standard_normal((cap, n_kv, hd)) * rng.uniform(0.5, 2, (cap, 1, 1))).astype(np.float32)
+    kq, vq = oracle_cache(oracle, k, v, np.arange(cap, dtype=np.int32), cap, 4, vbits)
+    q = rng.standard_normal((n_tok, n_kv, hd)).astype(np.float32)
+    en = (cap + cap // 2 + np.arange(n_tok)).astype(np.int32)
+    st = np.full(n_tok, en[-1] - cap + 1, np.int32)
+    scale = float(np.float32(1 / np.sqrt(hd)))
+    o = backend.kvq_attention(q, kq, vq, st, en, n_kv, 4, vbits, scale)
+    assert bits_equal(o, oracle_attention(oracle, q, kq, vq, st, en, n_kv, 4, vbits, scale))
