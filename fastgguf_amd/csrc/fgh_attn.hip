@@ -312,7 +312,7 @@ static void scores_launch(const AttnArgs &a, int n_tok, hipStream_t s) {
     else attn_scores16_kernel<HD, 4><<<g, 256, 0, s>>>(a, n_tok);
 }
 
-// scores of the per-row path (hd % 32 != 0): as attn_scores_kernel, thread = one key of the group's
+// scores of the per-row path (hd % 32 != 0): thread = one key of the group's
 // union, the q rows from LDS, K read value by value (any head size and offset), dot_f32v's order
 template <int R>
 __global__ __launch_bounds__(256) void attn_scores_row_kernel(AttnArgs a, int n_tok) {
@@ -1008,7 +1008,7 @@ hipError_t launch_attention(const AttnArgs &a, int n_tok, hipStream_t s) {
     else attn_softmax_kernel<256><<<rows, 256, lds, s>>>(a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return launch_attention_values(a, n_tok, s);  // 4 chains per lane from 64 rows per K / V head
+    return launch_attention_values(a, n_tok, s);
 }
 
 }  // namespace fgh
