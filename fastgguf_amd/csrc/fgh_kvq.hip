@@ -189,24 +189,46 @@ __global__ __launch_bounds__(64) void kvq_store_kernel(KvqStoreArgs a, int n_tok
     }
 }
 
-// the V scales of slot i % cap of K / V head i / cap, gathered: out[i]
+__device__ __forceinline__ int kvq_row_len(const KvqAttnArgs &a, int tok) {
+    const int n = a.en[tok] - a.st[tok] + 1;
+    return n >= 1 && n <= a.cap && n <= a.max_len ? n : 0;
+}
+
+// the V scales that some token's range reads, gathered: out[head * cap + slot]. A wavefront takes 64
+// slots of one head; lane t looks at tokens t, t + 64, .. for a range that meets them, and without one
+// nothing is read or written (a short range on a long ring would pay for every record of the cache).
 struct KvqGather {
-    const uint8_t *vq;
+    KvqAttnArgs a;
     float *out;  // null: none
-    int cap, n_head_kv, rec;
+    int n_tok;
+    unsigned wgs;  // workgroups, 4 wavefronts each
 };
+static unsigned kvq_gather_wgs(int cap, int n_head_kv) { return (unsigned)(((int64_t)((cap + 63) / 64) * n_head_kv + 3) / 4); }
+__device__ __forceinline__ void kvq_gather(const KvqGather &g) {
+    const KvqAttnArgs &a = g.a;
+    const int w = (int)blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int kvh = w % a.n_head_kv, s0 = w / a.n_head_kv * 64, sl = s0 + lane;
+    if (s0 >= a.cap) return;
+    bool used = false;
+    for (int t = lane; t < (g.n_tok + 63) / 64 * 64; t += 64) {  // uniform
+        if (t < g.n_tok) {
+            const int n = kvq_row_len(a, t), f = (int)slot_of(a.st[t], a.cap);  // slots f .. f + n - 1, around the ring
+            used = n > 0 && ((f < s0 + 64 && f + n > s0) || f + n - a.cap > s0);
+        }
+        if (__builtin_amdgcn_ballot_w64(used)) break;
+    }
+    if (!__builtin_amdgcn_ballot_w64(used) || sl >= a.cap) return;
+    const int rec = 4 + a.hd * a.vbits / 8;
+    g.out[(int64_t)kvh * a.cap + sl] = *(const float *)(a.vq + ((int64_t)sl * a.n_head_kv + kvh) * rec);
+}
 // rows of hd values rotated (inverse = false) or rotated back: one wavefront per row, 4 rows per
-// workgroup; the workgroups past them gather V scales
+// workgroup; the workgroups before them gather V scales
 __global__ __launch_bounds__(256) void kvq_rotate_kernel(const float *in, float *out, int hd, int rows, bool inverse, KvqGather g) {
-    const int nrot = (rows + 3) / 4;
-    if ((int)blockIdx.x >= nrot) {  // only launched with g.out
-        const int i = ((int)blockIdx.x - nrot) * 256 + threadIdx.x;
-        if (i >= g.cap * g.n_head_kv) return;
-        const int kvh = i / g.cap, sl = i - kvh * g.cap;
-        g.out[i] = *(const float *)(g.vq + ((int64_t)sl * g.n_head_kv + kvh) * g.rec);
+    if (blockIdx.x < g.wgs) {
+        kvq_gather(g);
         return;
     }
-    const int row = (int)blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int row = (int)(blockIdx.x - g.wgs) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= rows) return;
     float x[KVQ_E];
     row_load(x, in + (size_t)row * hd, hd);
@@ -214,11 +236,6 @@ __global__ __launch_bounds__(256) void kvq_rotate_kernel(const float *in, float 
 #pragma unroll
     for (int e = 0; e < KVQ_E; ++e)
         if (lane + 64 * e < hd) out[(size_t)row * hd + lane + 64 * e] = x[e];
-}
-
-__device__ __forceinline__ int kvq_row_len(const KvqAttnArgs &a, int tok) {
-    const int n = a.en[tok] - a.st[tok] + 1;
-    return n >= 1 && n <= a.cap && n <= a.max_len ? n : 0;
 }
 
 // Groups of R rows that read one K / V head kh: j = R q .. R q + R - 1 of the head's n_tok * G
@@ -454,17 +471,16 @@ hipError_t launch_kvq_attention(const KvqAttnArgs &a, int n_tok, hipStream_t s) 
         return hipErrorInvalidValue;
     const int rows_kv = n_tok * (a.n_head / a.n_head_kv);
     const unsigned kb = (unsigned)std::min((a.max_len + 255) / 256, 1024);
-    // prompt batches: every row reads its head's V scales, a cache line each out of the records. They
-    // are gathered once, into the scratch that the value chains fill later, where that holds them and
-    // the rows may read them 4 times and more (64 tokens, 32 heads, 4096 positions: the call 196.2 ->
-    // 186.3 us; 16 heads over 2, 1000 positions of 8-bit records 55.3 -> 52.6).
-    const KvqGather none{nullptr, nullptr, 0, 0, 0};
+    // prompt batches: every row reads its head's V scales, a cache line each out of the records. Those
+    // of the rows' ranges are gathered once, into the scratch that the value chains fill later, where
+    // that holds the ring's and the rows may read them 4 times and more (64 tokens, 32 heads, 4096
+    // positions: the call 196.2 -> 186.3 us; 16 heads over 2, 1000 positions of 8-bit records 55.3 -> 52.6).
     float *scales = nullptr;
     if (rows_kv >= 16) {
         const int64_t ns = (int64_t)a.n_head_kv * a.cap;
         if (ns <= (int64_t)rows * a.hd && 4 * ns <= (int64_t)rows * a.max_len && ns <= 0x3fffffff) scales = a.orot;
-        const KvqGather g{a.vq, scales, a.cap, a.n_head_kv, 4 + a.hd * a.vbits / 8};
-        kvq_rotate_kernel<<<(rows + 3) / 4 + (scales ? (unsigned)((ns + 255) / 256) : 0u), 256, 0, s>>>(a.q, a.qr, a.hd, rows, false, g);
+        const KvqGather g{a, scales, n_tok, scales ? kvq_gather_wgs(a.cap, a.n_head_kv) : 0u};
+        kvq_rotate_kernel<<<g.wgs + (unsigned)((rows + 3) / 4), 256, 0, s>>>(a.q, a.qr, a.hd, rows, false, g);
         kvq_scores_kernel<16><<<dim3(kb, (unsigned)((rows_kv + 15) / 16), (unsigned)a.n_head_kv), 256, 0, s>>>(a, n_tok);
     } else
         kvq_scores_kernel<4><<<dim3(kb, (unsigned)((rows_kv + 3) / 4), (unsigned)a.n_head_kv), 256, 0, s>>>(a, n_tok);
@@ -477,7 +493,7 @@ hipError_t launch_kvq_attention(const KvqAttnArgs &a, int n_tok, hipStream_t s) 
     v.vbits = a.vbits;
     hipError_t e = launch_attention_values(v, n_tok, s);
     if (e != hipSuccess) return e;
-    kvq_rotate_kernel<<<(rows + 3) / 4, 256, 0, s>>>(a.orot, a.o, a.hd, rows, true, none);
+    kvq_rotate_kernel<<<(rows + 3) / 4, 256, 0, s>>>(a.orot, a.o, a.hd, rows, true, KvqGather{a, nullptr, n_tok, 0u});
     return hipGetLastError();
 }
 
