@@ -258,7 +258,7 @@ __device__ __forceinline__ KvqRow kvq_group_row(const KvqAttnArgs &a, int n_tok,
     return g;
 }
 
-// scores: grid (key blocks, groups of R rows, K / V heads), 256 threads; thread = one key of the
+// scores: grid of key blocks, groups of R rows and K / V heads, 256 threads; thread = one key of the
 // group's union for its R rows: each record's codes are loaded and looked up once for R chains
 // in kvq_dot_k's order, then times s, times scale. R = 16 for prompt batches. R = 4 (decode): each
 // wavefront rotates one of the rows itself, while its keys' records are on their way: 10.8 us at 32
@@ -266,11 +266,18 @@ __device__ __forceinline__ KvqRow kvq_group_row(const KvqAttnArgs &a, int n_tok,
 // every key block would rotate 4 per wavefront.) A record's words are requested 8 ahead of their
 // use. Bound: latency, one or two wavefronts per CU and SIMD; twice the workgroups of 128 threads
 // took 11.5 us against 11.3.
+// The grid has key blocks for max_len keys; those past the range leave before they load a record.
+// R = 16: heads are the grid's fastest index, key blocks its slowest. With key blocks fastest the few
+// workgroups of a short range all went to one XCD (32 or 64 blocks a group, 8 XCDs in turn): 64 tokens x
+// 32 heads at the start of a ring of max_len 8192 took 77.9 us, now 38.2, and 4096 of 4096 positions
+// 180.8, now 177.9. R = 4 keeps key blocks fastest: a full range of 4096 positions is 54.2 us so (16
+// heads over 8, hd 256), 57.2 the other way.
 template <int R>
 __global__ __launch_bounds__(256) void kvq_scores_kernel(KvqAttnArgs a, int n_tok) {
     __shared__ float q[R][256];
     __shared__ float c4[16];
-    const int grp = blockIdx.y, kh = blockIdx.z, tid = threadIdx.x, hd = a.hd;
+    const int grp = blockIdx.y, kh = R == 16 ? blockIdx.x : blockIdx.z, tid = threadIdx.x, hd = a.hd;
+    const int kb = R == 16 ? blockIdx.z : blockIdx.x, nkb = R == 16 ? gridDim.z : gridDim.x;
     // every wavefront finds the group's ranges for itself: lane r (mod R) reads row r's, one round of
     // loads, and lane exchanges reduce them. R = 4: its own row of q is on its way meanwhile
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -288,7 +295,7 @@ __global__ __launch_bounds__(256) void kvq_scores_kernel(KvqAttnArgs a, int n_to
     }
     lo = __builtin_amdgcn_readfirstlane(lo);
     hi = __builtin_amdgcn_readfirstlane(hi);
-    if (hi < lo) return;
+    if (hi < lo || (int64_t)lo + (int64_t)kb * 256 > hi) return;  // the whole workgroup: no key of its own
     KvqRow rows[R];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -308,7 +315,7 @@ __global__ __launch_bounds__(256) void kvq_scores_kernel(KvqAttnArgs a, int n_to
         s = *(const float *)rp;
         words(cur, 0);
     };
-    int p = lo + (int)blockIdx.x * 256 + tid;
+    int p = lo + kb * 256 + tid;
     start(p);
     if constexpr (R == 4) {
         rotate_wave(x, hd, false);
@@ -323,7 +330,7 @@ __global__ __launch_bounds__(256) void kvq_scores_kernel(KvqAttnArgs a, int n_to
     }
     if (tid < 16) c4[tid] = kvq_centroid4(tid);
     __syncthreads();
-    for (; p <= hi; p += (int)gridDim.x * 256) {
+    for (; p <= hi; p += nkb * 256) {
         float acc[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) acc[r] = 0.0f;
@@ -360,7 +367,7 @@ __global__ __launch_bounds__(256) void kvq_scores_kernel(KvqAttnArgs a, int n_to
             const KvqRow g = rows[r];
             if (p >= g.st && p <= g.en) a.s[(size_t)g.row * a.max_len + (p - g.st)] = acc[r] * s * a.scale;
         }
-        if (p + (int)gridDim.x * 256 <= hi) start(p + (int)gridDim.x * 256);
+        if (p + nkb * 256 <= hi) start(p + nkb * 256);
     }
 }
 
@@ -481,7 +488,7 @@ hipError_t launch_kvq_attention(const KvqAttnArgs &a, int n_tok, hipStream_t s) 
         if (ns <= (int64_t)rows * a.hd && 4 * ns <= (int64_t)rows * a.max_len && ns <= 0x3fffffff) scales = a.orot;
         const KvqGather g{a, scales, n_tok, scales ? kvq_gather_wgs(a.cap, a.n_head_kv) : 0u};
         kvq_rotate_kernel<<<g.wgs + (unsigned)((rows + 3) / 4), 256, 0, s>>>(a.q, a.qr, a.hd, rows, false, g);
-        kvq_scores_kernel<16><<<dim3(kb, (unsigned)((rows_kv + 15) / 16), (unsigned)a.n_head_kv), 256, 0, s>>>(a, n_tok);
+        kvq_scores_kernel<16><<<dim3((unsigned)a.n_head_kv, (unsigned)((rows_kv + 15) / 16), kb), 256, 0, s>>>(a, n_tok);
     } else
         kvq_scores_kernel<4><<<dim3(kb, (unsigned)((rows_kv + 3) / 4), (unsigned)a.n_head_kv), 256, 0, s>>>(a, n_tok);
     const size_t lds = (size_t)std::min(a.max_len, KVQ_RES) * 4;

@@ -385,3 +385,9 @@ def test_prompt_cost_is_not_the_rings(backend):
     scales of slots outside every range are not read (read, they made the call 1.25 times as long;
     without, 1.02)."""
     assert ratio(backend, (16384, 1024), (1024, 1024)) < 1.12
+
+
+def test_prompt_cost_is_not_max_lens(backend):
+    """The same prompt batch with max_len 16384 costs little more than with 1024: the score launch's key
+    blocks past the range load nothing, and those with keys run on every XCD (3.4 times without)."""
+    assert ratio(backend, (16384, 16384), (16384, 1024)) < 1.8
