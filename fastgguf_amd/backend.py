@@ -31,7 +31,7 @@ EXPORTS = (
     "fgh_graph_begin", "fgh_graph_end", "fgh_graph_launch", "fgh_graph_destroy",
     "fgh_dev_alloc", "fgh_dev_free", "fgh_copy_h2d", "fgh_copy_d2h", "fgh_copy_d2d", "fgh_checksum_dev", "fgh_memcpy_dev", "fgh_mfma_peak_dev", "fgh_sync",
     "fgh_event_create", "fgh_event_record", "fgh_event_elapsed_ms", "fgh_event_destroy",
-    "fgh_quantize", "fgh_block_ints", "fgh_gemm_block_ints", "fgh_moe_block_ints", "fgh_expf", "fgh_fp16_to_f32", "fgh_matvec_shape",
+    "fgh_quantize", "fgh_block_ints", "fgh_gemm_block_ints", "fgh_moe_block_ints", "fgh_expf", "fgh_fp16_to_f32", "fgh_matvec_shape", "fgh_matmul_path",
     "fgh_gguf_open", "fgh_gguf_close", "fgh_gguf_summary", "fgh_gguf_tensor", "fgh_gguf_find",
     "fgh_gguf_kv_num", "fgh_gguf_kv_str", "fgh_gguf_data", "fgh_upload_gguf",
 )
@@ -114,6 +114,7 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
         "fgh_fp16_to_f32": (i32, [vp, vp, i32, vp]),
         "fgh_expf": (i32, [vp, f32p, i32, vp]),
         "fgh_matvec_shape": (i32, [vp, u32, i32, i64, i64, i32, vp]),
+        "fgh_matmul_path": (i32, [u32, i32, i64, i64, i64, i32, i32]),
         "fgh_gguf_open": (i32, [C.c_char_p, C.POINTER(vp), C.c_char_p, C.c_size_t]),
         "fgh_gguf_close": (None, [vp]),
         "fgh_gguf_summary": (i32, [vp, C.POINTER(u32), C.POINTER(u64), C.POINTER(i64), C.POINTER(i64)]),
@@ -134,6 +135,18 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
 
 def _p(a: np.ndarray):
     return a.ctypes.data_as(C.c_void_p)
+
+
+MATMUL_DECODE, MATMUL_GEMM, MATMUL_TOKENS = 0, 1, 2
+
+
+def matmul_path(ggml_type: int, order: int, cols: int, rows: int, ntok: int, n_mats: int = 1, num_cu: int = 256) -> int:
+    """The kernels that a matmul of ntok tokens runs (no device needed): MATMUL_DECODE per token,
+    MATMUL_GEMM, or MATMUL_TOKENS, which share a matrix's weights between tokens."""
+    rc = load_library().fgh_matmul_path(ggml_type, order, cols, rows, n_mats, ntok, num_cu)
+    if rc < 0:
+        raise BackendError(rc, "matmul_path: bad arguments")
+    return rc
 
 
 class Tensor:

@@ -379,13 +379,15 @@ static int gemm_q6k_into(fgh_ctx *c, const fgh_tensor *t, const float *X, int64_
 
 // the types and token counts that take a prompt GEMM (matmul, fastgguf.c:3018-3031), and the
 // activation-record bytes it needs (0: the per-token decode kernels, which need no scratch)
+static bool prompt_gemm_type(uint32_t type) {
+    return type == FGH_T_Q4_K || type == FGH_T_Q8_0 || type == FGH_T_Q6_K || q32n_type(type);
+}
 static size_t prompt_gemm_bytes(const fgh_ctx *c, const fgh_tensor *t, int T) {
-    if (T < 8) return 0;
+    if (T < 8 || !prompt_gemm_type(t->type)) return 0;
     if (t->type == FGH_T_Q4_K) return fgh::gemm_scratch(t->groups, t->nb, T, c->num_cu).bytes;
     if (t->type == FGH_T_Q8_0) return q80_scratch(c, t, T).bytes;
     if (t->type == FGH_T_Q6_K) return q6k_scratch(c, t, T).bytes;
-    if (q32n_type(t->type)) return fgh::gemmn_act_bytes(t->nb, (T + 15) / 16 * 16);
-    return 0;
+    return fgh::gemmn_act_bytes(t->nb, (T + 15) / 16 * 16);
 }
 // the prompt GEMM with its records in act (at least prompt_gemm_bytes)
 static int prompt_gemm_into(fgh_ctx *c, const fgh_tensor *t, const float *X, int64_t ldx, float *Y, int64_t ldy,
@@ -406,13 +408,13 @@ static int prompt_gemm(fgh_ctx *c, const fgh_tensor *t, const float *X, int64_t 
 // the kernels that share a matrix's weights between tokens, and the scratch bytes they need. Their
 // outputs are the per-token decode kernels' bit for bit, so a call whose scratch is not at hand
 // (a graph capture before any eager call) takes those.
-static bool tokens_path(const fgh_ctx *c, const fgh_tensor *t, int64_t ldx, int T) {
+static bool tokens_path(int num_cu, const fgh_tensor *t, int64_t ldx, int T) {
     if (T < 2) return false;
-    if (q16_rows(t->type)) return fgh::rowg_pays((int)t->type, t->order, t->groups, t->nb, T, c->num_cu);
+    if (q16_rows(t->type)) return fgh::rowg_pays((int)t->type, t->order, t->groups, t->nb, T, num_cu);
     if (!fgh::fl_kind((int)t->type)) return false;
     // the float kernels address X and a step of a matrix by 32-bit offsets
     return 4 * ((T - 1) * ldx + t->cols) <= 0x7fffffff && t->gpm * fgh::FL_TILE <= 0x7fffffff &&
-           fgh::fl_matmul_pays((int)t->type, t->rows * t->n_mats, (int)t->cols, T, c->num_cu);
+           fgh::fl_matmul_pays((int)t->type, t->rows * t->n_mats, (int)t->cols, T, num_cu);
 }
 static size_t tokens_bytes(const fgh_tensor *t, int T) { return q16_rows(t->type) ? fgh::rowg_act_bytes(t->nb, T) : 0; }
 static int tokens_into(fgh_ctx *c, const fgh_tensor *t, const float *X, int64_t ldx, float *Y, int64_t ldy, int T,
@@ -445,6 +447,21 @@ static int check_tensor(fgh_ctx *c, const fgh_tensor *t) {
     if (!c) return FGH_ERR_ARG;
     if (!t || t->ctx != c || !t->dev) return fail(c, FGH_ERR_ARG, "invalid tensor handle");
     return FGH_OK;
+}
+
+// the tile counts of a tensor of t's type and shape
+static void set_tiles(fgh_tensor *t) {
+    const uint32_t type = t->type;
+    t->nb = (int)(t->cols / block_elems(type));
+    t->ntile = fgh::fl_kind((int)type) ? (int)((t->cols + fgh::fl_step_elems((int)type) - 1) / fgh::fl_step_elems((int)type))
+               : fgh::q8_kind((int)type) ? (t->nb + 3) / 4
+                                          : t->nb;
+    const int tile_rows = q16_rows(type)               ? fgh::Q4K_TILE_ROWS
+                          : fgh::kq_kind((int)type) ? fgh::KQ_TILE_ROWS
+                          : fgh::fl_kind((int)type) ? fgh::fl_tile_rows((int)type)
+                                                    : 8;
+    t->gpm = (t->rows + tile_rows - 1) / tile_rows;
+    t->groups = t->gpm * t->n_mats;
 }
 
 extern "C" {
@@ -556,17 +573,8 @@ int fgh_upload(fgh_ctx *c, uint32_t type, int64_t cols, int64_t rows, int64_t n_
     t->cols = cols;
     t->rows = rows;
     t->n_mats = n_mats;
-    t->nb = (int)(cols / block_elems(type));
-    t->ntile = fgh::fl_kind((int)type) ? (int)((cols + fgh::fl_step_elems((int)type) - 1) / fgh::fl_step_elems((int)type))
-               : fgh::q8_kind((int)type) ? (t->nb + 3) / 4
-                                          : t->nb;
-    const int tile_rows = q16_rows(type)               ? fgh::Q4K_TILE_ROWS
-                          : fgh::kq_kind((int)type) ? fgh::KQ_TILE_ROWS
-                          : fgh::fl_kind((int)type) ? fgh::fl_tile_rows((int)type)
-                                                    : 8;
-    t->gpm = (rows + tile_rows - 1) / tile_rows;
-    t->groups = t->gpm * n_mats;
     t->order = ord;
+    set_tiles(t);
     int64_t dev_bytes = 0;
     if (__builtin_mul_overflow(t->groups, (int64_t)t->ntile * tile_bytes(type), &dev_bytes)) {
         delete t;
@@ -742,7 +750,7 @@ int fgh_matmul_dev(fgh_ctx *c, const fgh_tensor *t, const float *X, int ldx, flo
     // types Q4_0 / Q4_1 / Q5_0 / Q5_1; smaller batches, and the types without a GEMM in the reference,
     // keep the order of its token by token calls
     if (prompt_gemm_bytes(c, t, nb)) return prompt_gemm(c, t, X, ldx, Y, ldy, nb, nullptr, nullptr);
-    if (tokens_path(c, t, ldx, nb)) {
+    if (tokens_path(c->num_cu, t, ldx, nb)) {
         const size_t need = tokens_bytes(t, nb);
         if (!c->capturing || need <= c->gq.cap) {
             if ((rc = grow(c, c->gq, need))) return rc;
@@ -773,7 +781,7 @@ int fgh_matmul_dev_noalloc(fgh_ctx *c, const fgh_tensor *t, const float *X, int 
     if (gemm) return prompt_gemm_into(c, t, X, ldx, Y, ldy, nb, (uint8_t *)c->noalloc, nullptr, nullptr);
     // the several-token kernels that need scratch stay out: without a prompt GEMM a call here uses no
     // shared memory, so such calls may overlap
-    if (tokens_path(c, t, ldx, nb) && !tokens_bytes(t, nb)) return tokens_into(c, t, X, ldx, Y, ldy, nb, nullptr);
+    if (tokens_path(c->num_cu, t, ldx, nb) && !tokens_bytes(t, nb)) return tokens_into(c, t, X, ldx, Y, ldy, nb, nullptr);
     float *ys[1] = {Y};
     return matvec_launch(c, 1, &t, X, ldx, ys, ldy, nb, nullptr, nullptr);
 }
@@ -1467,6 +1475,21 @@ int fgh_matvec_shape(fgh_ctx *c, uint32_t type, int order, int64_t cols, int64_t
     shape[2] = sh.TPW;
     shape[3] = (int32_t)sh.lds;
     return FGH_OK;
+}
+
+int fgh_matmul_path(uint32_t type, int order, int64_t cols, int64_t rows, int64_t n_mats, int ntok, int num_cu) {
+    if (!type_supported(type) || cols < 1 || rows < 1 || n_mats < 1 || ntok < 1 || ntok > FG_BATCH || num_cu < 1 ||
+        cols % block_elems(type) != 0)
+        return FGH_ERR_ARG;
+    fgh_tensor t = {};
+    t.type = type;
+    t.cols = cols;
+    t.rows = rows;
+    t.n_mats = n_mats;
+    t.order = type == FGH_T_Q4_K && order == FGH_ORDER_REPACKED ? FGH_ORDER_REPACKED : FGH_ORDER_ROW;
+    set_tiles(&t);
+    if (ntok >= 8 && prompt_gemm_type(type)) return FGH_MATMUL_GEMM;
+    return tokens_path(num_cu, &t, cols, ntok) ? FGH_MATMUL_TOKENS : FGH_MATMUL_DECODE;
 }
 
 int fgh_expf(fgh_ctx *c, const float *x, int n, float *out) {

@@ -392,21 +392,39 @@ hipError_t rg_launch_type(const RgArgs &a, int num_cu, hipStream_t s) {
 
 size_t rowg_act_bytes(int nb, int T) { return (size_t)((T + 15) / 16) * nb * (RG_FRAG + RG_SMALL); }
 
-// Whether these kernels take less time than the per-token decode launches, from what both measured on
-// MI355X (us): the decode launches 4 + (0.057 Q4_K repacked, 0.055 Q4_K row order, 0.078 Q5_K) per
-// token and million weights (14336 x 4096: Q4_K 5 tokens 20.5, Q5_K 64 tokens 297; 1024 x 4096 Q5_K
-// 33 tokens 16.8), since they split a short matrix's blocks over wavefronts; these 6 + a block time
-// (0.57 one group of Q4_K repacked, 0.78 in row order; 0.98 for several groups apart, 1.9 for two per wavefront)
-// times the blocks of a row and the rounds of wavefronts, since a row's blocks are walked by one
-// (15.5 and 35.5 for the first two, 21 for the third; 4096 x 14336 Q4_K 4 tokens 36.7 against 17.4).
+// Whether these kernels take less time than the per-token decode launches: both sides from what they
+// measured on MI355X (us; 1138 calls: 36 shapes from 512 x 2048 to 3584 x 18944 and 50000 x 768, 2..7
+// tokens, Q5_K 2..64). The decode launches walk a row's blocks in rounds of one wavefront per SIMD (a
+// tile and token each; shorter launches split their tiles and are never slower), and read a matrix
+// beyond 64 MiB anew for every token. These walk all blocks of a row in one wavefront, up to two per SIMD.
+//                                   decode -> these     rule        decode -> these     rule
+//   Q4_K repacked  14336 x 4096   4 16.7   16.6  decode   5 20.0   16.4  these
+//   Q4_K row order 14336 x 4096   4 18.7   19.4  decode   5 21.5   19.2  these
+//   Q4_K repacked   8192 x 8192   6 20.7   24.1  decode   7 25.3   24.2  these
+//   Q5_K           14336 x 4096   4 20.8   23.6  decode   5 24.4   23.5  these
+//   Q5_K            4096 x 14336 12 46.9   62.1  decode  17 71.7   60.4  these
+//   Q5_K            1024 x 4096  64 18.9   22.0  decode
+//   Q5_K           14336 x 4096                          64 263.2  36.3  these
+// In none of those calls it picks these kernels where they are more than 2.5 % slower; in 6 it keeps
+// decode launches that are 8 to 27 % slower (Q4_K 28672 x 4096 at 3 tokens the most).
 bool rowg_pays(int type, int order, int64_t groups, int nb, int T, int num_cu) {
-    const double mw = groups * 16.0 * nb * 256.0 * 1e-6;
-    const double before = 4 + T * mw * (type == T_Q5_K ? 0.078 : order == 1 ? 0.057 : 0.055);
+    struct Fit {
+        double base, block, round_block, round, far, one, one2;
+    };
+    const Fit f = type == T_Q5_K ? Fit{2.3, 0.171, 0.188, 0.55, 1.65, 0.97, 1.6}
+                  : order == 1   ? Fit{3.05, 0.057, 0.167, 0.33, 1.48, 0.54, 1.07}
+                                 : Fit{2.9, 0.139, 0.18, 0.23, 1.4, 0.72, 1.2};
+    const int64_t simds = 4 * (int64_t)num_cu;
+    const bool far = groups * nb * (type == T_Q5_K ? Q5K_TILE : Q4K_TILE) > (int64_t)64 << 20;
+    const double rounds = (double)((groups * T + simds - 1) / simds);
+    const double before = f.base + f.block * nb + rounds * (f.round_block * (far ? f.far : 1.0) * nb + f.round);
     const int tg = (T + 15) / 16;
     const bool two = tg > 1 && (groups + 3) / 4 * ((tg + 1) / 2) >= num_cu * 3 / 4;
-    const int64_t waves = groups * (two ? (tg + 1) / 2 : tg), slots = (two ? 8 : 4) * (int64_t)num_cu;
-    const double block = two ? 1.9 : tg > 1 ? 0.98 : order == 1 ? 0.57 : 0.78;
-    return before > 1.1 * (6 + block * nb * ((waves + slots - 1) / slots));
+    const int64_t waves = groups * (two ? (tg + 1) / 2 : tg);
+    const double one = two ? 1.17 : tg > 1 ? 0.95 : f.one;    // a block, at up to one wavefront per SIMD
+    const double more = two ? 1.7 : tg > 1 ? 1.43 : f.one2;  // and at up to two, for each such round
+    const double block = waves <= simds ? one : more * (double)((waves + 2 * simds - 1) / (2 * simds));
+    return before > (two ? 8.0 : 6.6) + block * nb;
 }
 
 hipError_t launch_rowg(int type, int order, const RowgArgs &r, int num_cu, hipStream_t s) {

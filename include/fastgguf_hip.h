@@ -340,7 +340,14 @@ FGH_API int fgh_event_destroy(fgh_ctx *ctx, void *ev);
  * IQ4_XS, 4 for F32, 8 for F16, 64 for BF16, 8 otherwise) and ntok tokens picks: shape[0]
  * wavefronts per tile, [1] ring depth, [2]
  * tiles per workgroup, [3]
- * LDS bytes. Lets the tests run every kernel instantiation the launchers can choose. */
+ * LDS bytes. Lets the tests run every kernel instantiation the launchers can choose.
+ * fgh_matmul_path: the kernels that fgh_matmul of ntok tokens (X rows cols apart) runs on a device of
+ * num_cu compute units for n_mats matrices of rows x cols (order as fgh_upload resolved it):
+ * FGH_MATMUL_DECODE the decode launches per token, FGH_MATMUL_GEMM the prompt GEMM, FGH_MATMUL_TOKENS
+ * the kernels that share a matrix's weights between tokens. Needs no device. */
+#define FGH_MATMUL_DECODE 0
+#define FGH_MATMUL_GEMM 1
+#define FGH_MATMUL_TOKENS 2
 FGH_API int fgh_quantize(fgh_ctx *ctx, int kind, const float *x, int n, void *out_blocks);
 FGH_API int fgh_block_ints(fgh_ctx *ctx, const fgh_tensor *t, const float *x, int32_t *sumi, int32_t *msum);
 FGH_API int fgh_gemm_block_ints(fgh_ctx *ctx, const fgh_tensor *t, const float *X, int ldx, int nb,
@@ -357,6 +364,7 @@ FGH_API int fgh_expf(fgh_ctx *ctx, const float *x, int n, float *out);
 FGH_API int fgh_fp16_to_f32(fgh_ctx *ctx, const uint16_t *h, int n, float *out);
 FGH_API int fgh_matvec_shape(fgh_ctx *ctx, uint32_t type, int order, int64_t cols, int64_t row_tiles, int ntok,
                              int32_t *shape);
+FGH_API int fgh_matmul_path(uint32_t type, int order, int64_t cols, int64_t rows, int64_t n_mats, int ntok, int num_cu);
 
 #ifdef __cplusplus
 }
