@@ -642,6 +642,13 @@ struct RowgArgs {
     int64_t rows, gpm, groups, ldx, ldy;
     int nb, T;         // blocks (float types: values) per row, tokens
 };
+// MiB of a matrix that one XCD's L2 (4 MiB) meets in a per-token decode launch of wgs workgroups per
+// token: workgroups go to the 8 XCDs in turn, so a row's are all on one XCD if wgs is a multiple of 8
+// and on 8 / gcd otherwise. It sets what the tokens after the first read from the L2.
+inline double decode_l2_mib(double bytes, int64_t wgs) {
+    const int gcd = wgs % 8 == 0 ? 8 : wgs % 4 == 0 ? 4 : wgs % 2 == 0 ? 2 : 1;
+    return bytes / gcd / (1 << 20);
+}
 size_t rowg_act_bytes(int nb, int T);
 bool rowg_pays(int type, int order, int64_t groups, int nb, int T, int num_cu);  // faster than the per-token launches
 bool fl_matmul_pays(int type, int64_t rows, int n, int T, int num_cu);

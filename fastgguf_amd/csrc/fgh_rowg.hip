@@ -393,29 +393,31 @@ hipError_t rg_launch_type(const RgArgs &a, int num_cu, hipStream_t s) {
 size_t rowg_act_bytes(int nb, int T) { return (size_t)((T + 15) / 16) * nb * (RG_FRAG + RG_SMALL); }
 
 // Whether these kernels take less time than the per-token decode launches: both sides from what they
-// measured on MI355X (us; 1138 calls: 36 shapes from 512 x 2048 to 3584 x 18944 and 50000 x 768, 2..7
+// measured on MI355X (us; 1740 calls: 62 shapes from 512 x 2048 to 3584 x 18944 and 60851 x 256, 2..7
 // tokens, Q5_K 2..64). The decode launches walk a row's blocks in rounds of one wavefront per SIMD (a
-// tile and token each; shorter launches split their tiles and are never slower), and read a matrix
-// beyond 64 MiB anew for every token. These walk all blocks of a row in one wavefront, up to two per SIMD.
+// tile and token each; shorter launches split their tiles and are never slower), more slowly where an XCD's
+// L2 doesn't hold its share of the matrix for the next token. These walk all blocks of a row in one
+// wavefront, up to two per SIMD.
 //                                   decode -> these     rule        decode -> these     rule
 //   Q4_K repacked  14336 x 4096   4 16.7   16.6  decode   5 20.0   16.4  these
 //   Q4_K row order 14336 x 4096   4 18.7   19.4  decode   5 21.5   19.2  these
 //   Q4_K repacked   8192 x 8192   6 20.7   24.1  decode   7 25.3   24.2  these
 //   Q5_K           14336 x 4096   4 20.8   23.6  decode   5 24.4   23.5  these
+//   Q5_K           12464 x 5888   3 28.1   30.2  decode   5 41.2   29.9  these
 //   Q5_K            4096 x 14336 12 46.9   62.1  decode  17 71.7   60.4  these
 //   Q5_K            1024 x 4096  64 18.9   22.0  decode
 //   Q5_K           14336 x 4096                          64 263.2  36.3  these
-// In none of those calls it picks these kernels where they are more than 2.5 % slower; in 6 it keeps
-// decode launches that are 8 to 27 % slower (Q4_K 28672 x 4096 at 3 tokens the most).
+// In one of those calls it picks these kernels where they are 4 % slower, in none more; in 10 it keeps decode
+// launches that are 8 to 18 % slower.
 bool rowg_pays(int type, int order, int64_t groups, int nb, int T, int num_cu) {
     struct Fit {
         double base, block, round_block, round, far, one, one2;
     };
-    const Fit f = type == T_Q5_K ? Fit{2.3, 0.171, 0.188, 0.55, 1.65, 0.97, 1.6}
-                  : order == 1   ? Fit{3.05, 0.057, 0.167, 0.33, 1.48, 0.54, 1.07}
-                                 : Fit{2.9, 0.139, 0.18, 0.23, 1.4, 0.72, 1.2};
+    const Fit f = type == T_Q5_K ? Fit{2.4, 0.051, 0.216, 0.462, 1.373, 0.97, 1.6}
+                  : order == 1   ? Fit{2.265, 0.079, 0.175, 0.262, 1.185, 0.54, 1.07}
+                                 : Fit{2.68, 0.229, 0.151, 0.32, 1.275, 0.72, 1.2};
     const int64_t simds = 4 * (int64_t)num_cu;
-    const bool far = groups * nb * (type == T_Q5_K ? Q5K_TILE : Q4K_TILE) > (int64_t)64 << 20;
+    const bool far = decode_l2_mib((double)groups * nb * (type == T_Q5_K ? Q5K_TILE : Q4K_TILE), (groups + 3) / 4) > 5.8;
     const double rounds = (double)((groups * T + simds - 1) / simds);
     const double before = f.base + f.block * nb + rounds * (f.round_block * (far ? f.far : 1.0) * nb + f.round);
     const int tg = (T + 15) / 16;

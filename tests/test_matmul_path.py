@@ -22,6 +22,7 @@ MEASURED = [
     (S.T_Q5_K, ROW, 8192, 2048, 8, 11.6, 14.9), (S.T_Q5_K, ROW, 1024, 4096, 64, 18.9, 22.0),
     (S.T_Q5_K, ROW, 4096, 1536, 16, 10.2, 12.7), (S.T_Q5_K, ROW, 2048, 2048, 64, 19.4, 14.3),
     (S.T_Q5_K, ROW, 16376, 1024, 5, 9.4, 10.7), (S.T_Q5_K, ROW, 16376, 1024, 16, 22.2, 10.8),
+    (S.T_Q5_K, ROW, 12464, 5888, 3, 28.1, 30.2), (S.T_Q5_K, ROW, 12464, 5888, 5, 41.2, 29.9),
 ]
 
 
