@@ -563,21 +563,42 @@ static int fl_mm_nt(int type, int64_t groups, int tg, int num_cu) {
     while (nt > 1 && (groups + 3) / 4 * ((tg + nt - 1) / nt) < num_cu * 3 / 4) nt >>= 1;
     return nt;
 }
-// Whether these kernels take less time than the per-token decode launches, from what both measured on
-// MI355X (us, n values a row): the decode launches 3 + (F32 0.5, F16 0.13 below 8 M weights and 0.19
-// above) per token and million weights, BF16 the larger of 0.0113 n and 0.155 per token and
-// million; these 4 + (F32 0.48, F16 0.375 per group of tokens) per 64 values, BF16 0.026 per
-// value, times the rounds of wavefronts (a wavefront walks its whole rows). 14336 x 2048, 64
-// tokens: F32 998 -> 72, F16 444 -> 52, BF16 312 -> 58; 4096 x 4096: 533 -> 38, 195 -> 31, 152 -> 107.
+// Whether these kernels take less time than the per-token decode launches: both sides from what they
+// measured on MI355X (us; 1012 calls a type: 59 shapes from 256 x 256 to 11008 x 4096, 151936 x 128 and
+// 602 x 12608, 2..64 tokens). The decode launches take a wavefront per tile and token: a part per tile, the
+// scalar tail, and one per value that grows with what an XCD's L2 meets of the matrix, up to 2 MiB and again
+// to 8 (F16 3120 x 4192, 98 workgroups a token: 16 tokens 55.8; 4096 x 4096, 128 of them: 38.4). These walk a
+// row in one wavefront: rounds of one per SIMD.
+//                        decode -> these   rule           decode -> these   rule
+//   F32   640 x 2048   40  15.6   20.0  decode
+//   F32   512 x 4096   40  22.0   34.5  decode
+//   F32  4096 x 4096    4  33.0   35.9  decode      8  65.2   36.0  these
+//   F32 14336 x 2048                                64 991.1   69.9  these
+//   F16  3072 x 3072   14  18.2   22.9  decode     24  25.2   22.8  these
+//   F16 14336 x 2048                                64 379.4   50.2  these
+//   BF16 4096 x 4096   48 100.2  107.1  decode     64 139.2  107.4  these
+//   BF16 14336 x 2048   8  39.3   56.9  decode     64 291.8   56.8  these
+// In three of those calls it picks these kernels where they are 3 % slower, in none more; in 36 it keeps
+// decode launches that are 8 to 43 % slower (BF16 16400 x 1024 at 8 tokens the most).
 bool fl_matmul_pays(int type, int64_t rows, int n, int T, int num_cu) {
-    const double mw = (double)rows * n * 1e-6;
+    struct Fit {
+        double base, chain, tile, value, l2, far, tail;  // chain, value, l2, far: per 1000 values of a row
+    };
+    const Fit f = type == T_F32   ? Fit{2.8, 0.08, 0.711, 0.333, 0.52, 0.78, 0.57}
+                  : type == T_F16 ? Fit{2.6, 1.4, 0.57, 0.35, 0.12, 0.78, 0.5}
+                                  : Fit{2.85, 0.8, 1.0, 2.8, 1.6, 7.27, 0.1};
+    const double simds = 4.0 * num_cu, k = n / 1000.0;
+    const int64_t tiles = (rows + fl_tile_rows(type) - 1) / fl_tile_rows(type);
+    const int tpw = fl_matvec_shape(type, tiles * T, n, num_cu).TPW;
+    const double mib = decode_l2_mib((double)rows * n * (type == T_F32 ? 4 : 2), (tiles + tpw - 1) / tpw);
+    const double value = f.value + f.l2 * std::min(mib, 2.0) / 2 + f.far * (std::min(std::max(mib, 2.0), 8.0) - 2) / 6;
+    const double before = f.base + f.chain * k + tiles * T / simds * (value * k + f.tile + (n % 8 ? f.tail : 0.0));
     const int tg = (T + 15) / 16;
     const int64_t groups = (rows + (type == T_BF16 ? 63 : 15)) / (type == T_BF16 ? 64 : 16);
     const int nt = fl_mm_nt(type, groups, tg, num_cu);
     const double rounds = (double)((groups * ((tg + nt - 1) / nt) + 4 * num_cu - 1) / (4 * num_cu));
-    if (type == T_BF16) return std::max(0.0113 * n, 0.155 * T * mw) > 1.15 * (2 + 0.026 * n * rounds);
-    const double before = 3 + T * mw * (type == T_F32 ? 0.5 : mw < 8 ? 0.13 : 0.19);
-    return before > 1.15 * (4 + (type == T_F32 ? 0.48 : 0.375 * nt) * ((n + 63) / 64) * rounds);
+    if (type == T_BF16) return before > 3 + rounds * (1 + 0.0258 * n);
+    return before > 3 + rounds * (1 + (type == T_F32 ? 0.48 : 0.375 * nt) * ((n + 63) / 64)) + (n % 8 ? 2.5 : 0.0);
 }
 template <int TYPE>
 static hipError_t fl_mm_launch(const FlMmArgs &a, int num_cu, hipStream_t s) {

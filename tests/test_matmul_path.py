@@ -23,6 +23,16 @@ MEASURED = [
     (S.T_Q5_K, ROW, 4096, 1536, 16, 10.2, 12.7), (S.T_Q5_K, ROW, 2048, 2048, 64, 19.4, 14.3),
     (S.T_Q5_K, ROW, 16376, 1024, 5, 9.4, 10.7), (S.T_Q5_K, ROW, 16376, 1024, 16, 22.2, 10.8),
     (S.T_Q5_K, ROW, 12464, 5888, 3, 28.1, 30.2), (S.T_Q5_K, ROW, 12464, 5888, 5, 41.2, 29.9),
+    (S.T_F32, ROW, 640, 2048, 40, 15.6, 20.0), (S.T_F32, ROW, 512, 4096, 64, 29.7, 34.6),
+    (S.T_F32, ROW, 896, 4864, 28, 35.0, 41.4), (S.T_F32, ROW, 1024, 1024, 20, 9.1, 12.4),
+    (S.T_F32, ROW, 4096, 4096, 4, 33.0, 35.9), (S.T_F32, ROW, 4096, 4096, 8, 65.2, 36.0),
+    (S.T_F32, ROW, 14336, 2048, 64, 991.1, 69.9), (S.T_F32, ROW, 1003, 1003, 64, 35.5, 14.2),
+    (S.T_F16, ROW, 3072, 3072, 14, 18.2, 22.9), (S.T_F16, ROW, 3072, 3072, 32, 30.6, 23.0),
+    (S.T_F16, ROW, 1024, 4096, 64, 25.5, 28.9), (S.T_F16, ROW, 1536, 8960, 24, 47.7, 57.1),
+    (S.T_F16, ROW, 14336, 2048, 64, 379.4, 50.2), (S.T_F16, ROW, 2048, 512, 64, 20.9, 8.2),
+    (S.T_F16, ROW, 3120, 4192, 16, 55.8, 29.7), (S.T_F16, ROW, 4096, 4096, 12, 29.8, 28.9),
+    (S.T_BF16, ROW, 4096, 4096, 48, 100.2, 107.1), (S.T_BF16, ROW, 4096, 4096, 64, 139.2, 107.4),
+    (S.T_BF16, ROW, 14336, 2048, 8, 39.3, 56.9), (S.T_BF16, ROW, 14336, 2048, 64, 291.8, 56.8),
 ]
 
 
