@@ -179,3 +179,71 @@ def test_attention_value_tile_edges(backend, oracle, n_tok, n_head, n_kv, hd, le
     scale = float(np.float32(1 / np.sqrt(hd)))
     o = backend.attention(q, ck, cv, st, en, n_kv, scale)
     assert bits_equal(o, oracle_attention(oracle, q, ck, cv, st, en, n_kv, scale))
+
+
+# rows per K head (token x query heads of the K head): the 4-row score kernel up to 15, the 16-row one with 1, 2
+# and 4 wavefronts from 16, 17 and 33; the 16-row value kernel from 64
+@pytest.mark.parametrize("n_tok,g", [(1, 1), (5, 3), (4, 4), (17, 1), (8, 4), (11, 3), (16, 4), (13, 5)], ids=lambda v: str(v))
+@pytest.mark.parametrize("hd", [32, 64, 96, 128, 160, 192, 224, 256])
+def test_attention_score_kernel_forms(backend, oracle, hd, n_tok, g):
+    """Every head size of the vector path in every score kernel form, ranges that end around its 64-key
+    tiles (63, 64, 65 and 130 keys for the first token) over a ring that wraps inside one, two K heads."""
+    rng = np.random.default_rng(hd + 7 * n_tok + g)
+    n_kv = 2
+    scale = float(np.float32(1 / np.sqrt(hd)))
+    for length in (63, 64, 65, 130):
+        cap = length + n_tok + 2
+        ck = rng.standard_normal((cap, n_kv * hd)).astype(np.float32)
+        cv = rng.standard_normal((cap, n_kv * hd)).astype(np.float32)
+        q = rng.standard_normal((n_tok, g * n_kv, hd)).astype(np.float32)
+        st = np.full(n_tok, cap - 20, np.int32)
+        en = (st + length - 1 + np.arange(n_tok)).astype(np.int32)
+        o = backend.attention(q, ck, cv, st, en, n_kv, scale)
+        assert bits_equal(o, oracle_attention(oracle, q, ck, cv, st, en, n_kv, scale)), length
+
+
+@pytest.mark.parametrize("n_tok,n_head", [(1, 2), (65, 4)], ids=["1024_threads", "256_threads"])
+@pytest.mark.parametrize("length", [12288, 12289, 12300, 2 * 12288 + 5])
+def test_attention_rows_beyond_lds(backend, oracle, n_tok, n_head, length):
+    """Rows around and past the softmax's 12,288 resident positions (longer ones go through LDS in
+    chunks that carry the ordered lane sums), in both of its workgroup sizes."""
+    rng = np.random.default_rng(length + n_tok)
+    hd, cap = 32, length + n_tok
+    ck = rng.standard_normal((cap, hd)).astype(np.float32)
+    cv = rng.standard_normal((cap, hd)).astype(np.float32)
+    q = (rng.standard_normal((n_tok, n_head, hd)) * 2).astype(np.float32)
+    st = np.full(n_tok, 77, np.int32)
+    en = (st + length - 1).astype(np.int32)
+    en[-1] += n_tok > 1
+    scale = float(np.float32(1 / np.sqrt(hd)))
+    o = backend.attention(q, ck, cv, st, en, 1, scale)
+    assert bits_equal(o, oracle_attention(oracle, q, ck, cv, st, en, 1, scale))
+
+
+@pytest.mark.parametrize("n_tok,g", [(2, 2), (4, 4), (16, 2), (20, 4)], ids=["scores4_values4", "scores16_1", "scores16_2", "scores16_4_values16"])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_attention_mfma_specials(backend, oracle, hd, n_tok, g):
+    """The fp32 MFMAs add each product as one fmaf: scores of subnormal products (scaled back up), -inf
+    scores from an infinity in K, and value sums over subnormals, infinities and NaN in V. All rows
+    attend the same positions; outputs equal bit for bit, any NaN as any NaN."""
+    rng = np.random.default_rng(hd + n_tok)
+    n = 150
+    q = rng.standard_normal((n_tok, g, hd)).astype(np.float32)
+    q[..., 5] = np.abs(q[..., 5])
+    ck = rng.standard_normal((n, hd)).astype(np.float32)
+    cv = rng.standard_normal((n, hd)).astype(np.float32)
+    ck[7, 5] = ck[90, 5] = -np.inf
+    cv[:, 1] *= np.float32(1e-39)
+    cv[:, 2] = np.float32(1e-44)
+    cv[:, 3] = -0.0
+    cv[100, 8], cv[101, 9] = np.inf, -np.inf
+    cv[3, 10], cv[140, 10] = np.inf, -np.inf
+    cv[77, 11] = np.nan
+    st, en = np.zeros(n_tok, np.int32), np.full(n_tok, n - 1, np.int32)
+    for qs, ks, scale in ((1.0, 1.0, float(np.float32(1 / np.sqrt(hd)))), (1e-20, 1e-20, 3e38)):
+        qq, kk = (q * np.float32(qs)).astype(np.float32), (ck * np.float32(ks)).astype(np.float32)
+        o = backend.attention(qq, kk, cv, st, en, 1, scale)
+        want = oracle_attention(oracle, qq, kk, cv, st, en, 1, scale)
+        assert np.isnan(want[..., 10:12]).all() and np.isinf(want[..., 8:10]).all()
+        assert np.isfinite(want[..., 12:]).all() and np.abs(want[..., 1]).max() < 1.2e-38
+        assert bits_equal_or_nan(o, want)
