@@ -330,6 +330,46 @@ def test_attention_prompt_scattered_ranges(backend, oracle, cap, n_tok):
     assert bits_equal(o, oracle_attention(oracle, q, kq, vq, st, en, n_kv, 4, 4, scale))
 
 
+def random_cache(rng, cap, n_kv, hd, bits, top):
+    """Records of random codes with positive finite scales up to top."""
+    c = rng.integers(0, 256, (cap, n_kv * rec_bytes(hd, bits)), dtype=np.uint8)
+    for h in range(n_kv):
+        at = h * rec_bytes(hd, bits)
+        c[:, at:at + 4] = rng.uniform(top / 4, top, (cap, 1)).astype(np.float32).view(np.uint8)
+    return c
+
+
+@pytest.mark.parametrize("cap", [1200, 5120, 5200])
+@pytest.mark.parametrize("length", [255, 1023, 1025, 1100])
+def test_attention_many_rows(backend, oracle, cap, length):
+    """More than 256 rows (the softmax's 256-thread form): ranges below and past the 4 x 256 positions whose
+    V scales it holds ahead, the scales gathered (2 heads x cap <= 320 rows x 32) and read from the records."""
+    rng = np.random.default_rng(cap + length)
+    n_tok, n_head, n_kv, hd = 40, 8, 2, 32
+    kq, vq = random_cache(rng, cap, n_kv, hd, 4, 0.1), random_cache(rng, cap, n_kv, hd, 4, 2.0)
+    q = rng.standard_normal((n_tok, n_head, hd)).astype(np.float32)
+    st = np.full(n_tok, cap - 300, np.int32)
+    en = (st + length - 1 + np.arange(n_tok)).astype(np.int32)
+    scale = float(np.float32(1 / np.sqrt(hd)))
+    o = backend.kvq_attention(q, kq, vq, st, en, n_kv, 4, 4, scale)
+    assert bits_equal(o, oracle_attention(oracle, q, kq, vq, st, en, n_kv, 4, 4, scale))
+
+
+@pytest.mark.parametrize("n_tok,n_head", [(1, 2), (65, 4)], ids=["1024_threads", "256_threads"])
+@pytest.mark.parametrize("length", [12288, 12289, 12300])
+def test_attention_rows_beyond_lds(backend, oracle, n_tok, n_head, length):
+    """Rows around and past the softmax's 12,288 resident positions, in both of its workgroup sizes."""
+    rng = np.random.default_rng(length + n_tok)
+    hd, cap = 32, length + n_tok
+    kq, vq = random_cache(rng, cap, 1, hd, 8, 0.002), random_cache(rng, cap, 1, hd, 2, 2.0)
+    q = rng.standard_normal((n_tok, n_head, hd)).astype(np.float32)
+    st = np.full(n_tok, 77, np.int32)
+    en = (st + length - 1).astype(np.int32)
+    scale = float(np.float32(1 / np.sqrt(hd)))
+    o = backend.kvq_attention(q, kq, vq, st, en, 1, 8, 2, scale)
+    assert bits_equal(o, oracle_attention(oracle, q, kq, vq, st, en, 1, 8, 2, scale))
+
+
 def prompt_us(backend, cap, max_len, shape=(64, 64, 64, 256), bits=(8, 8)):
     """A function timing one TurboQuant prompt call over the first 64 positions of a cap-slot ring: us a
     call in one replay of a graph of 10 (and the function freeing its buffers)."""
