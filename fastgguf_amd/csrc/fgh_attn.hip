@@ -23,8 +23,6 @@
 // pointers; other head sizes read K and (when a 16-byte read would not be aligned) V value by value.
 #include <hip/hip_runtime.h>
 
-#include <utility>
-
 #include "fgh_internal.h"
 
 namespace fgh {
@@ -48,9 +46,6 @@ __device__ __forceinline__ float exp_neg_ref(float x) {
     const float e = __builtin_bit_cast(float, (uint32_t)((int)fx + 127) << 23);
     return keep ? y * e : 0.0f;
 }
-
-__device__ __forceinline__ float f_xor1(float v) { return __builtin_bit_cast(float, dpp_xor1(__builtin_bit_cast(int, v))); }
-__device__ __forceinline__ float f_xor2(float v) { return __builtin_bit_cast(float, dpp_xor2(__builtin_bit_cast(int, v))); }
 
 // the rows' ranges: n = en - st + 1, or 0 when the range is empty, longer than the cache or than
 // the score buffer (such a row gets NaN outputs)
@@ -82,7 +77,7 @@ __device__ __forceinline__ GroupRow group_row(const AttnArgs &a, int n_tok, int 
     return g;
 }
 // A group's ranges, found by every wavefront for itself: lane r (mod R) reads row r's range, so the
-// group costs one round of loads, and lane exchanges reduce them. R: 4 or 16.
+// group costs one round of loads, and lane exchanges reduce them. R: 4, 16, 32 or 64.
 struct GroupSpan {
     int lo, hi;        // the union of the rows' ranges; hi < lo: none is valid
     int in_lo, in_hi;  // the positions inside every valid row's range
@@ -125,13 +120,8 @@ typedef float av4u __attribute__((ext_vector_type(4), aligned(4)));  // a 16-byt
 // ---- scores ----
 // K = 1 MFMAs run the 8 lane chains: chain l of every (row, key) pair of a tile is one accumulator
 // register set, and dimension d adds q_d k_d to chain d % 8, each as one fmaf, dimension after
-// dimension (measured bit for bit, as the value kernels). K tiles of 64 keys go through LDS: 1 KB
-// loads of whole rows in, one 16-byte read of 4 dimensions per key out.
-// f(integral_constant 0), f(integral_constant 1), ...: an MFMA's broadcast block is an immediate
-template <class F, int... J>
-__device__ __forceinline__ void for_seq(F &&f, std::integer_sequence<int, J...>) {
-    (f(std::integral_constant<int, J>{}), ...);
-}
+// dimension (subnormals, infinities and NaN included; the tests compare bits, as for the values). K tiles
+// of 64 keys go through LDS: 1 KB loads of whole rows in, one 16-byte read of 4 dimensions per key out.
 
 // K rows of positions p0 .. p0 + 63 (past hi: hi's row) into dst[64][HD + 4], NT threads: pieces
 // j B .. j B + B - 1 of each thread
@@ -183,7 +173,9 @@ __device__ __forceinline__ float chain_tree(float a0, float a1, float a2, float 
 // dimension's block to all four), B = K (lane = key), 8 chains x 16 registers of sums, in flight
 // one after another. The next tile's loads are in flight
 // in registers while a tile is multiplied (head sizes up to 128).
-// Bound: one 32-cycle MFMA per dimension and 16 rows x 64 keys.
+// 64 tokens x 32 heads over 8, 4096 positions, hd 128: 35 us. One 32-cycle MFMA per dimension and 16
+// rows x 64 keys is about 15 of them (counters: the matrix pipe is busy 32.8 k cycles a SIMD); with two
+// wavefronts a SIMD the rest is the range search, the q loads, the tiles' two barriers and the epilogue.
 template <int HD, int NW>
 __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 192 ? 2 : 1) void attn_scores16_kernel(AttnArgs a, int n_tok) {
     __shared__ __attribute__((aligned(16))) float kt[64 * (HD + 4)];
@@ -248,8 +240,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && HD <= 192 ? 2 : 1) void attn_sc
 // scores of fewer rows (decode): grid (K heads, key chunks), 2 wavefronts that work alone. A wavefront
 // takes a tile of 64 keys into its own part of LDS and multiplies it with the head's rows, 4 at a
 // time, by v_mfma_f32_4x4x1 (one register holds 16 dimensions x 4 rows of q): K is read once
-// whatever the rows. Bound: K's bytes from HBM (all tiles of a 4096-position decode step are in
-// flight at once).
+// whatever the rows. 32 heads over 8, 4096 positions, hd 128: 6.7 us; K's bytes are 2.5 of them. Every tile
+// is in flight at once, two wavefronts a CU: a wavefront's one pass bounds it, 43 % of its life waits
+// for its tile and 36 % issues VALU work (1667 instructions: addresses, LDS stores, the trees).
 template <int HD>
 __global__ __launch_bounds__(128) void attn_scores4_kernel(AttnArgs a, int n_tok) {
     __shared__ __attribute__((aligned(16))) float kt[2][64 * (HD + 4)];
@@ -644,8 +637,8 @@ struct AvWeights {
 // values of prompt batches: grid (K heads, groups of 16 rows, 64-column chunks), 4 chain wavefronts
 // and 8 loading wavefronts. Chain wavefront w sums rows 4 w .. 4 w + 3 of the group over the
 // chunk's 64 columns with v_mfma_f32_4x4x1: its 16 blocks are 16 groups of 4 columns, K = 1 is one
-// position, so one instruction adds w_p v_p to 256 sums, each as one fmaf (measured bit for bit on
-// 8 M random products, subnormals, infinities and NaN included), in the position's turn. cbsz = 4
+// position, so one instruction adds w_p v_p to 256 sums, each as one fmaf (subnormals, infinities and
+// NaN included), in the position's turn. cbsz = 4
 // broadcasts one of 16 blocks of the weight register to all: one register holds 16 positions x 4
 // rows, one LDS read. The reads of 16 positions are issued before the MFMAs of the 16 before them,
 // one wait per batch. The loaders hold 4 tiles of 128 positions in flight in registers (all
@@ -655,8 +648,11 @@ struct AvWeights {
 // only its own positions st..en, so a position of another row of the group adds nothing to it (not
 // even fma(0, v, acc), which is NaN for a non-finite v and turns -0 into +0); the vector path's
 // att_v_kern walks the group's whole span with zero weights, as the chains do without PR
-// Bound: one dependent MFMA per position, 12.2 cycles (15.2 with the LDS reads of 4 wavefronts per
-// CU), one wavefront per SIMD at 64 tokens x 32 heads, hd 128.
+// 64 tokens x 32 heads over 8, 4096 positions, hd 128: 50 us, 1.5 (3200 to 3600 cycles) a tile. The chain,
+// one dependent MFMA of 12.2 cycles per position, is 1560 of them, 1950 with the LDS reads of 4 wavefronts
+// a CU. By the counters the LDS is active for a third of the time (a quarter of that bank conflicts) and the
+// matrix pipe for less: neither is the bound; all wavefronts together spend half their cycles in waits
+// (the tile's barrier, loads, LDS).
 constexpr int AP_T = 128, AP_P = AP_T + 4, AP_W = AP_T + 16;  // positions per tile, LDS rows of V and of the weights
 template <int VB, bool SC, bool PR>
 __global__ __launch_bounds__(768) void attn_values16_kernel(AttnArgs a, int n_tok) {
@@ -820,7 +816,9 @@ __device__ __forceinline__ void fmac16_bcast(float &acc, float w, const av4 &a, 
 // LDS ([column][position]), so one 16-byte read feeds 4 positions and the 4 rows share it; the
 // row's weight comes in by a lane broadcast inside the fma. The reads of the next 32 positions
 // are issued before the 32 fmas of the current ones, one wait for the whole batch.
-// Bound: 4096 dependent fmas per lane (about 5.3 cycles each, 7 with the reads).
+// 32 heads over 8, 4096 positions, hd 128: 18.5 us. 4096 dependent fmas per lane are 9 to 12 of them (about
+// 5.3 cycles each, 7 with the reads); the rest is the range search, the first tiles' way from memory
+// and the loaders' stores (a quarter of the LDS cycles are bank conflicts).
 constexpr int AD_T = 256, AD_P = AD_T + 4;  // positions per tile, LDS row (16 columns of 16 bytes cover all banks)
 template <int VB, bool SC, bool PR>
 __global__ __launch_bounds__(320) void attn_values4_kernel(AttnArgs a, int n_tok) {

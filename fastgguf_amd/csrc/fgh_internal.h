@@ -6,6 +6,8 @@
 #include <limits.h>
 #include <stdint.h>
 
+#include <utility>
+
 namespace fgh {
 
 // ---------------------------------------------------------------------------------------------
@@ -110,6 +112,12 @@ __device__ __forceinline__ int q8_round(float v) {
 }
 __device__ __forceinline__ uint32_t pack_q(int a, int b, int c, int d) {
     return (uint32_t)(a & 0xFF) | ((uint32_t)(b & 0xFF) << 8) | ((uint32_t)(c & 0xFF) << 16) | ((uint32_t)(d & 0xFF) << 24);
+}
+
+// f(integral_constant 0), f(integral_constant 1), ...: an MFMA's broadcast block is an immediate
+template <class F, int... J>
+__device__ __forceinline__ void for_seq(F &&f, std::integer_sequence<int, J...>) {
+    (f(std::integral_constant<int, J>{}), ...);
 }
 
 // the workgroup's barrier after LDS writes and reads: global loads stay in flight

@@ -4,11 +4,12 @@
 // Records: one per (slot, K / V head), KVQ_REC = 4 + hd * bits / 8 bytes: the float scale, then
 // the codes (8 bits: int8; 4 bits: low nibble first; 2 bits: low bits first). A slot holds the
 // n_head_kv records of one position back to back. The rotation R x = H(D x) / sqrt(hd) (signs D
-// of xorshift64*, kvq_init 3363-3372; butterflies kvq_fwht 3375-3386) is done in LDS, one
-// butterfly per thread per stage, so every value sees the reference's additions.
+// of xorshift64*, kvq_init 3363-3372; butterflies kvq_fwht 3375-3386) of a row runs in one wavefront by
+// lane exchanges (rotate_wave), so every value sees the reference's additions.
 //
 // Attention (hd a power of 2, 32..256):
-//   q rows rotated (4763)                                    kvq_rotate_kernel
+//   q rows rotated (4763)                                    kvq_rotate_kernel (16 rows and more per
+//                                                            K / V head), else in kvq_scores_kernel
 //   scores: kvq_dot_k (3447-3462) times scale, per key       kvq_scores_kernel
 //   softmax_inplace (3147-3156), then w' = w * s_V(p)         kvq_softmax_kernel
 //   o = fma(w', centroid, o) over the positions in order     attn_values (fgh_attn.hip), which
@@ -264,8 +265,8 @@ __device__ __forceinline__ KvqRow kvq_group_row(const KvqAttnArgs &a, int n_tok,
 // wavefront rotates one of the rows itself, while its keys' records are on their way: 10.8 us at 32
 // heads, 4096 positions, hd 128, against 9.7 and a rotation launch of 4.0. (With 16 rows per group
 // every key block would rotate 4 per wavefront.) A record's words are requested 8 ahead of their
-// use. Bound: latency, one or two wavefronts per CU and SIMD; twice the workgroups of 128 threads
-// took 11.5 us against 11.3.
+// use. Bound at decode: latency, 128 workgroups of one wavefront a SIMD, which waits for half of its life;
+// twice the workgroups of 128 threads took 11.5 us against 11.3.
 // The grid has key blocks for max_len keys; those past the range leave before they load a record.
 // R = 16: heads are the grid's fastest index, key blocks its slowest. With key blocks fastest the few
 // workgroups of a short range all went to one XCD (32 or 64 blocks a group, 8 XCDs in turn): 64 tokens x

@@ -30,9 +30,10 @@
 // once per wavefront (about 130 VALU instructions, Q5_K 230, against 56 per group); with 4 groups
 // the 192 chain registers would lie in accumulation registers, two moves for every fma (measured:
 // 49.7 us).
-// Bound: VALU issue; at one group the weight stream.
-#include <utility>
-
+// Bound (counters): two groups, Q5_K 14336 x 4096, 64 tokens (31 us after a quantizer launch of 4): VALU
+// issue, 42.7 k of the 63.5 k cycles that a SIMD is busy (matrix pipe 10.8 k). One group, Q4_K, 5 tokens (12 us
+// after a launch of 3.5): the latency of a block's steps in the one wavefront of a SIMD, which issues for half
+// of its life, waits a third of it for results of MFMAs and fmas and a sixth for memory.
 #include "fgh_internal.h"
 
 namespace fgh {
@@ -137,11 +138,6 @@ __device__ __forceinline__ h8 rg_operand(uint32_t q, uint32_t M, uint32_t F, uin
     const h2 a = __builtin_elementwise_fma(as_h2(l02), sl, ol), b = __builtin_elementwise_fma(as_h2(h02), sh, oh);
     const h2 c = __builtin_elementwise_fma(as_h2(l13), sl, ol), e = __builtin_elementwise_fma(as_h2(h13), sh, oh);
     return (h8){a.x, a.y, b.x, b.y, c.x, c.y, e.x, e.y};
-}
-
-template <class Fn, int... I>
-__device__ __forceinline__ void for_ints(Fn &&f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
 }
 
 struct RgArgs {
@@ -288,13 +284,13 @@ __global__ __launch_bounds__(256, 2) void rowg_kernel(RgArgs a) {
         };
         if constexpr (NG == 1) {
             scales();
-            for_ints([&](auto kk) {
+            for_seq([&](auto kk) {
                 constexpr int k = decltype(kk)::value;
                 add(kk, 0, f.a[k], rg_operand<TYPE, k>(q[k], M, F, E, fl, fh, sl, ol, sh, oh));
             }, std::make_integer_sequence<int, 8>{});
         } else {
             scales();
-            for_ints([&](auto kk) {
+            for_seq([&](auto kk) {
                 constexpr int k = decltype(kk)::value;
                 const h8 Bk = rg_operand<TYPE, k>(q[k], M, F, E, fl, fh, sl, ol, sh, oh);
 #pragma unroll

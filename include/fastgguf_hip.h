@@ -229,8 +229,9 @@ FGH_API int fgh_matmul_dev(fgh_ctx *ctx, const fgh_tensor *t, const float *X_dev
 /* fgh_matmul_dev without any device allocation. No counterpart in the reference: it is for
  * callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc). From nb >= 8 tokens the prompt GEMM's scratch goes to a static device
- * array of FGH_NOALLOC_SCRATCH_BYTES per device, held until the process ends (under 8 tokens the
- * decode kernels run and need none). Its size per type, Tp = nb rounded up to 16 (Q8_0: 32 or 64):
+ * array of FGH_NOALLOC_SCRATCH_BYTES per device, held until the process ends (under 8 tokens, and for
+ * types without a prompt GEMM, the decode kernels or the float types' several-token kernels run and need
+ * none). Its size per type, Tp = nb rounded up to 16 (Q8_0: 32 or 64):
  *   Q4_K, Q6_K  (256-blocks + 1) * 292 * Tp bytes of activation records;
  *   Q8_0        (steps + KH) * 144 * Tp bytes of records, steps = ceil(32-blocks / 4), KH = 4
  *               from 4 steps (2 for 2-3 steps, 1 for one);
