@@ -407,7 +407,7 @@ static int prompt_gemm(fgh_ctx *c, const fgh_tensor *t, const float *X, int64_t 
 // The matmuls of several tokens that the reference runs token by token, in its row kernels' orders:
 // the kernels that share a matrix's weights between tokens, and the scratch bytes they need. Their
 // outputs are the per-token decode kernels' bit for bit, so a call whose scratch is not at hand
-// (a graph capture before any eager call) takes those.
+// (a graph capture before any eager call, a full card) takes those.
 static bool tokens_path(int num_cu, const fgh_tensor *t, int64_t ldx, int T) {
     if (T < 2) return false;
     if (q16_rows(t->type)) return fgh::rowg_pays((int)t->type, t->order, t->groups, t->nb, T, num_cu);
@@ -752,10 +752,9 @@ int fgh_matmul_dev(fgh_ctx *c, const fgh_tensor *t, const float *X, int ldx, flo
     if (prompt_gemm_bytes(c, t, nb)) return prompt_gemm(c, t, X, ldx, Y, ldy, nb, nullptr, nullptr);
     if (tokens_path(c->num_cu, t, ldx, nb)) {
         const size_t need = tokens_bytes(t, nb);
-        if (!c->capturing || need <= c->gq.cap) {
-            if ((rc = grow(c, c->gq, need))) return rc;
+        if (need <= c->gq.cap || (!c->capturing && grow(c, c->gq, need) == FGH_OK))
             return tokens_into(c, t, X, ldx, Y, ldy, nb, (uint8_t *)c->gq.p);
-        }
+        (void)hipGetLastError();  // no memory for the scratch: the decode launches need none
     }
     float *ys[1] = {Y};
     return matvec_launch(c, 1, &t, X, ldx, ys, ldy, nb, nullptr, nullptr);

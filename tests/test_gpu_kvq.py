@@ -414,7 +414,7 @@ def prompt_us(backend, cap, max_len, shape=(64, 64, 64, 256), bits=(8, 8)):
 def ratio(backend, a, b):
     """The fastest replay of prompt call a over the fastest of b, timed in turn."""
     (ua, fa), (ub, fb) = prompt_us(backend, *a), prompt_us(backend, *b)
-    times = [(ua(), ub()) for _ in range(12)][2:]
+    times = [(ua(), ub()) for _ in range(30)][2:]
     fa()
     fb()
     return min(t[0] for t in times) / min(t[1] for t in times)
