@@ -8,8 +8,8 @@
 // lane exchanges (rotate_wave), so every value sees the reference's additions.
 //
 // Attention (hd a power of 2, 32..256):
-//   q rows rotated (4763)                                    kvq_rotate_kernel (16 rows and more per
-//                                                            K / V head), else in kvq_scores_kernel
+//   q rows rotated (4763)                                    kvq_rotate_gather_kernel (16 rows and
+//                                                            more per K / V head), else in kvq_scores_kernel
 //   scores: kvq_dot_k (3447-3462) times scale, per key       kvq_scores_kernel
 //   softmax_inplace (3147-3156), then w' = w * s_V(p)         kvq_softmax_kernel
 //   o = fma(w', centroid, o) over the positions in order     attn_values (fgh_attn.hip), which
@@ -223,13 +223,9 @@ __device__ __forceinline__ void kvq_gather(const KvqGather &g) {
     g.out[(int64_t)kvh * a.cap + sl] = *(const float *)(a.vq + ((int64_t)sl * a.n_head_kv + kvh) * rec);
 }
 // rows of hd values rotated (inverse = false) or rotated back: one wavefront per row, 4 rows per
-// workgroup; the workgroups before them gather V scales
-__global__ __launch_bounds__(256) void kvq_rotate_kernel(const float *in, float *out, int hd, int rows, bool inverse, KvqGather g) {
-    if (blockIdx.x < g.wgs) {
-        kvq_gather(g);
-        return;
-    }
-    const int row = (int)(blockIdx.x - g.wgs) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+// workgroup
+__device__ __forceinline__ void rotate_rows(const float *in, float *out, int hd, int rows, bool inverse, unsigned wg) {
+    const int row = (int)wg * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= rows) return;
     float x[KVQ_E];
     row_load(x, in + (size_t)row * hd, hd);
@@ -237,6 +233,14 @@ __global__ __launch_bounds__(256) void kvq_rotate_kernel(const float *in, float 
 #pragma unroll
     for (int e = 0; e < KVQ_E; ++e)
         if (lane + 64 * e < hd) out[(size_t)row * hd + lane + 64 * e] = x[e];
+}
+__global__ __launch_bounds__(256) void kvq_rotate_kernel(const float *in, float *out, int hd, int rows, bool inverse) {
+    rotate_rows(in, out, hd, rows, inverse, blockIdx.x);
+}
+// the query rows rotated; the first g.wgs workgroups gather V scales
+__global__ __launch_bounds__(256) void kvq_rotate_gather_kernel(KvqGather g) {
+    if (blockIdx.x < g.wgs) kvq_gather(g);
+    else rotate_rows(g.a.q, g.a.qr, g.a.hd, g.n_tok * g.a.n_head, false, blockIdx.x - g.wgs);
 }
 
 // Groups of R rows that read one K / V head kh: j = R q .. R q + R - 1 of the head's n_tok * G
@@ -488,7 +492,7 @@ hipError_t launch_kvq_attention(const KvqAttnArgs &a, int n_tok, hipStream_t s) 
         const int64_t ns = (int64_t)a.n_head_kv * a.cap;
         if (ns <= (int64_t)rows * a.hd && 4 * ns <= (int64_t)rows * a.max_len && ns <= 0x3fffffff) scales = a.orot;
         const KvqGather g{a, scales, n_tok, scales ? kvq_gather_wgs(a.cap, a.n_head_kv) : 0u};
-        kvq_rotate_kernel<<<g.wgs + (unsigned)((rows + 3) / 4), 256, 0, s>>>(a.q, a.qr, a.hd, rows, false, g);
+        kvq_rotate_gather_kernel<<<g.wgs + (unsigned)((rows + 3) / 4), 256, 0, s>>>(g);
         kvq_scores_kernel<16><<<dim3((unsigned)a.n_head_kv, (unsigned)((rows_kv + 15) / 16), kb), 256, 0, s>>>(a, n_tok);
     } else
         kvq_scores_kernel<4><<<dim3(kb, (unsigned)((rows_kv + 3) / 4), (unsigned)a.n_head_kv), 256, 0, s>>>(a, n_tok);
@@ -501,7 +505,7 @@ hipError_t launch_kvq_attention(const KvqAttnArgs &a, int n_tok, hipStream_t s) 
     v.vbits = a.vbits;
     hipError_t e = launch_attention_values(v, n_tok, s);
     if (e != hipSuccess) return e;
-    kvq_rotate_kernel<<<(rows + 3) / 4, 256, 0, s>>>(a.orot, a.o, a.hd, rows, true, KvqGather{a, nullptr, n_tok, 0u});
+    kvq_rotate_kernel<<<(rows + 3) / 4, 256, 0, s>>>(a.orot, a.o, a.hd, rows, true);
     return hipGetLastError();
 }
 
